@@ -118,6 +118,228 @@ __global__ __launch_bounds__(256) void wvb_q8_kernel(WvbArgs a) {
         reinterpret_cast<float *>(reinterpret_cast<char *>(a.dst) + (size_t)t * a.d_nb1 + (size_t)h * a.d_nb2)[o] = acc;
 }
 
+// ---- several tokens (chunked prefill): wv_b and WKB as tiled products ----
+// The per-token kernels above re-read the head's weights and re-quantise its activations for every
+// few outputs of every token.  From Q8_GEMM_MIN_TOKENS tokens on a workgroup takes 32 tokens of one
+// head and quantises them once, into LDS.
+constexpr int Q8_GEMM_MIN_TOKENS = 16;
+constexpr int GT = 32;                   // tokens per workgroup
+constexpr uint32_t Q_PAD = 16;           // LDS row padding: rows start on distinct banks
+
+struct __attribute__((packed, aligned(4))) F4u { float v[4]; };       // 16 bytes at dword alignment
+struct __attribute__((packed, aligned(4))) U4u { uint32_t v[4]; };
+
+// Half a Q8 block of token r = lane & 31 (values 16 (lane >> 5) .. +15 of the block at x): its int8
+// quants as 4 dwords and the block's scale, with quant_lane's arithmetic (the two halves of a block
+// meet by v_permlane32_swap).
+template <bool DIV>
+__device__ __forceinline__ u32x4 quant_half_block(const F4u (&x)[4], float & d16) {
+    float amax = fabsf(x[0].v[0]);
+#pragma unroll
+    for (int i = 1; i < 16; ++i) amax = fmaxf(amax, fabsf(x[i >> 2].v[i & 3]));
+    float lo, hi;
+    halves_pair(amax, lo, hi);
+    amax = fmaxf(lo, hi);
+    const float d = amax / 127.0f;
+    d16 = round_to_f16(d);
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t wv = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = x[i].v[e];
+            int q;
+            if constexpr (DIV) q = amax == 0.0f ? 0 : (int)roundf(v / d);
+            else q = (int)roundf(v * id);
+            wv |= ((uint32_t)(uint8_t)(int8_t)q) << (8 * e);
+        }
+        r[i] = wv;
+    }
+    return r;
+}
+
+// The 16 int8 of half kh of block b of a Q8_0 row (4-byte aligned, an even number of blocks): the
+// qs start 2 bytes past a dword in even blocks (a fifth dword, still inside the row, is read) and
+// on one in odd blocks.
+__device__ __forceinline__ u32x4 q8_half_block(const uint8_t * row, int b, int kh) {
+    const uint8_t * p = row + 34 * b + 16 * kh;
+    if (b & 1) {
+        const U4u u = *reinterpret_cast<const U4u *>(p + 2);
+        return u32x4{u.v[0], u.v[1], u.v[2], u.v[3]};
+    }
+    const U4u u = *reinterpret_cast<const U4u *>(p);
+    const uint32_t e = *reinterpret_cast<const uint32_t *>(p + 16);
+    return u32x4{__builtin_amdgcn_alignbyte(u.v[1], u.v[0], 2), __builtin_amdgcn_alignbyte(u.v[2], u.v[1], 2),
+                 __builtin_amdgcn_alignbyte(u.v[3], u.v[2], 2), __builtin_amdgcn_alignbyte(e, u.v[3], 2)};
+}
+__device__ __forceinline__ float q8_value(const u32x4 & q, int j, float d) {
+    return (float)(int)(int8_t)(uint8_t)(q[j >> 2] >> (8 * (j & 3))) * d;
+}
+
+// Quantise GT tokens of head h (rows of NB blocks at x + t x_nbt): the workgroup's waves take blocks
+// w, w + 4, ...; quants to xq[token][NB * 32 + Q_PAD], scales to xd[block][token].
+template <int NB, bool DIV>
+__device__ __forceinline__ void quant_tokens(const char * x, int64_t x_nbt, int t0, int nt, char * xq, float (*xd)[GT]) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = lane & 31, kh = lane >> 5;
+    const float * row = reinterpret_cast<const float *>(x + (size_t)min(t0 + r, nt - 1) * x_nbt) + 16 * kh;
+    constexpr int BPW = (NB + 3) / 4;
+    F4u v[BPW][4];
+#pragma unroll
+    for (int i = 0; i < BPW; ++i)
+        if (w + 4 * i < NB) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[i][k] = *reinterpret_cast<const F4u *>(row + 32 * (w + 4 * i) + 4 * k);
+        }
+#pragma unroll
+    for (int i = 0; i < BPW; ++i) {
+        const int b = w + 4 * i;
+        if (b < NB) {
+            float d16;
+            const u32x4 q = quant_half_block<DIV>(v[i], d16);
+            *reinterpret_cast<u32x4 *>(xq + r * (NB * 32 + Q_PAD) + 32 * b + 16 * kh) = q;
+            if (kh == 0) xd[b][r] = d16;
+        }
+    }
+}
+
+// wv_b over 32 tokens x 128 outputs of one head: wave w takes outputs 32 w .. +31.
+// The per-token kernel's result is, per element position k of a block, a chain over the blocks of
+// fma(wd_b xd_b, qw qx, .), then the butterfly over k.  wd_b xd_b (two f16 scales), qw wd_b and
+// qx xd_b are exact in f32, so each link is also fma(qw wd_b, qx xd_b, .): an outer product over
+// (token, output) per (k, b), which v_mfma_f32_32x32x1_2b_f32 (K = 1: one fused multiply-add per
+// element) computes with the same single rounding.  Its two blocks take positions j and j + 16, whose
+// sums are the butterfly's first step; the other steps are additions of accumulators in the
+// butterfly's order (16, 8, 4, 2, 1), so the result is the per-token kernel's bit for bit.
+// Bound: 2 x 16 NB MFMAs of 64 cycles per SIMD at two waves (NB = 8: 6.8 us for the 1,024 waves
+// of 512 tokens x 32 heads).
+template <int NB>
+__global__ __launch_bounds__(256, NB <= 8 ? 2 : 1) void wvb_q8_gemm_kernel(WvbArgs a) {
+    static_assert(NB % 2 == 0 && NB >= 4, "rows of an even number of blocks are 4-byte aligned");
+    __shared__ __attribute__((aligned(16))) char xq[GT * (NB * 32 + Q_PAD)];
+    __shared__ float xd[NB][GT];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = lane & 31, kh = lane >> 5;
+    const int t0 = blockIdx.x * GT, o0 = blockIdx.y * 128 + 32 * w, h = blockIdx.z;
+    // B operand: column o0 + r, element positions 16 kh + j of every block
+    const uint8_t * wrow = a.w + ((size_t)h * a.d_out + min(o0 + r, a.d_out - 1)) * (NB * 34);
+    u32x4 qw[NB];
+    float wd[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        qw[b] = q8_half_block(wrow, b, kh);
+        wd[b] = f16_bits(*reinterpret_cast<const uint16_t *>(wrow + 34 * b));
+    }
+    quant_tokens<NB, false>(reinterpret_cast<const char *>(a.x) + (size_t)h * a.x_nb2, a.x_nb1, t0, a.nt, xq, xd);
+    __syncthreads();
+    if (o0 >= a.d_out) return;               // whole waves leave together
+    // A operand: token t0 + r, the same element positions
+    u32x4 qx[NB];
+    float xs[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        qx[b] = *reinterpret_cast<const u32x4 *>(xq + r * (NB * 32 + Q_PAD) + 32 * b + 16 * kh);
+        xs[b] = xd[b][r];
+    }
+    typedef float f32x32 __attribute__((ext_vector_type(32)));
+    // positions j, j + 16, j + 8 and j + 24 of the block: two chains, then the first two butterfly steps
+    auto s8 = [&](int j) __attribute__((always_inline)) {
+        f32x32 c0, c1;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) { c0[i] = 0.0f; c1[i] = 0.0f; }
+        // the operands of block b + 1 are converted under the MFMAs of block b; the scheduling
+        // barriers keep the compiler from converting every block first (and spilling)
+        float xa = q8_value(qx[0], j, xs[0]), xb = q8_value(qx[0], j + 8, xs[0]);
+        float ya = q8_value(qw[0], j, wd[0]), yb = q8_value(qw[0], j + 8, wd[0]);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            c0 = __builtin_amdgcn_mfma_f32_32x32x1f32(xa, ya, c0, 0, 0, 0);
+            c1 = __builtin_amdgcn_mfma_f32_32x32x1f32(xb, yb, c1, 0, 0, 0);
+            if (b + 1 < NB) {
+                xa = q8_value(qx[b + 1], j, xs[b + 1]);
+                xb = q8_value(qx[b + 1], j + 8, xs[b + 1]);
+                ya = q8_value(qw[b + 1], j, wd[b + 1]);
+                yb = q8_value(qw[b + 1], j + 8, wd[b + 1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = (c0[i] + c0[16 + i]) + (c1[i] + c1[16 + i]);
+        asm volatile("" : "+v"(s));          // added here: left alone, the additions sink and both chains spill
+        return s;
+    };
+    auto s4 = [&](int j) __attribute__((always_inline)) { f32x16 x = s8(j); x = x + s8(j + 4); asm volatile("" : "+v"(x)); return x; };
+    auto s2 = [&](int j) __attribute__((always_inline)) { f32x16 x = s4(j); x = x + s4(j + 2); asm volatile("" : "+v"(x)); return x; };
+    f32x16 s = s2(0);
+    s = s + s2(1);
+    // row of register i: token 8 (i / 4) + 4 (lane >> 5) + (i & 3); column: output lane & 31
+    const int o = o0 + r;
+    if (o >= a.d_out) return;
+    char * d = reinterpret_cast<char *>(a.dst) + (size_t)h * a.d_nb2 + 4 * (size_t)o;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int t = t0 + 8 * (i >> 2) + 4 * kh + (i & 3);
+        if (t < a.nt) *reinterpret_cast<float *>(d + (size_t)t * a.d_nb1) = s[i];
+    }
+}
+
+// WKB over 32 tokens of one head, every output: wave w takes 32-column blocks w, w + 4, ...  The
+// int32 dot of one Q8 block is one v_mfma_i32_32x32x32_i8 (exact), then acc = fma(wd * d16, sum,
+// acc) over the blocks in order, the per-token kernel's operations bit for bit.
+template <int NB>
+__global__ __launch_bounds__(256) void wkb_q8_gemm_kernel(WkbArgs a) {
+    typedef int i32x16 __attribute__((ext_vector_type(16)));
+    __shared__ __attribute__((aligned(16))) char xq[GT * (NB * 32 + Q_PAD)];
+    __shared__ __attribute__((aligned(16))) float xd[NB][GT];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = lane & 31, kh = lane >> 5;
+    const int h = blockIdx.x, t0 = blockIdx.y * GT;
+    quant_tokens<NB, true>(reinterpret_cast<const char *>(a.q) + (size_t)h * a.q_nb1, a.q_nb2, t0, a.nt, xq, xd);
+    __syncthreads();
+    i32x4 qx[NB];
+    f32x4 xs[NB][4];                         // scales of this lane's 16 result rows (tokens)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        qx[b] = *reinterpret_cast<const i32x4 *>(xq + r * (NB * 32 + Q_PAD) + 32 * b + 16 * kh);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xs[b][i] = *reinterpret_cast<const f32x4 *>(&xd[b][8 * i + 4 * kh]);
+    }
+    for (int c0 = 32 * w; c0 < a.d_v; c0 += 128) {
+        const int c = c0 + r;
+        const uint8_t * wrow = a.wq + ((size_t)h * a.d_v + min(c, a.d_v - 1)) * (NB * 34);
+        u32x4 qw[NB];
+        float wd[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            qw[b] = q8_half_block(wrow, b, kh);
+            wd[b] = f16_bits(*reinterpret_cast<const uint16_t *>(wrow + 34 * b));
+        }
+        f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            i32x16 s;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 0;
+            s = __builtin_amdgcn_mfma_i32_32x32x32_i8(qx[b], __builtin_bit_cast(i32x4, qw[b]), s, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] = fmaf(wd[b] * xs[b][i >> 2][i & 3], (float)s[i], acc[i]);
+        }
+        if (c < a.d_v) {
+            char * d = reinterpret_cast<char *>(a.dst) + (size_t)h * a.d_nb1 + 4 * (size_t)c;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int t = t0 + 8 * (i >> 2) + 4 * kh + (i & 3);
+                if (t < a.nt) *reinterpret_cast<float *>(d + (size_t)t * a.d_nb2) = acc[i];
+            }
+        }
+    }
+}
+
 // ---- PHASE 0, KV-write ----
 // gemv: a workgroup per output row, a thread per 32-value block of the input (m4-phase.cu:95-125):
 // the thread quantises its block itself, acc = (wd * d16) * sum, the butterfly per 32 blocks, then
@@ -249,6 +471,13 @@ __global__ __launch_bounds__(1024) void kvwrite_tail_kernel(KvWriteArgs a) {
 }  // namespace
 
 hipError_t launch_wkb_q8(const WkbArgs & a, hipStream_t stream) {
+    if (a.nt >= Q8_GEMM_MIN_TOKENS) {
+        const dim3 grid(a.n_head, (a.nt + GT - 1) / GT);
+        if (a.d_n == 64) hipLaunchKernelGGL(wkb_q8_gemm_kernel<2>, grid, dim3(256), 0, stream, a);
+        else if (a.d_n == 128) hipLaunchKernelGGL(wkb_q8_gemm_kernel<4>, grid, dim3(256), 0, stream, a);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
     const dim3 grid(a.n_head, a.nt);
     if (a.d_n == 64) hipLaunchKernelGGL(wkb_q8_kernel<2>, grid, dim3(256), 0, stream, a);
     else if (a.d_n == 128) hipLaunchKernelGGL(wkb_q8_kernel<4>, grid, dim3(256), 0, stream, a);
@@ -257,6 +486,13 @@ hipError_t launch_wkb_q8(const WkbArgs & a, hipStream_t stream) {
 }
 
 hipError_t launch_wvb_q8(const WvbArgs & a, hipStream_t stream) {
+    if (a.nt >= Q8_GEMM_MIN_TOKENS) {
+        const dim3 grid((a.nt + GT - 1) / GT, (a.d_out + 127) / 128, a.n_head);
+        if (a.d_in == 256) hipLaunchKernelGGL(wvb_q8_gemm_kernel<8>, grid, dim3(256), 0, stream, a);
+        else if (a.d_in == 512) hipLaunchKernelGGL(wvb_q8_gemm_kernel<16>, grid, dim3(256), 0, stream, a);
+        else return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
     const dim3 grid((a.d_out + 7) / 8, a.n_head, a.nt);
     if (a.d_in == 256) hipLaunchKernelGGL(wvb_q8_kernel<8>, grid, dim3(256), 0, stream, a);
     else if (a.d_in == 512) hipLaunchKernelGGL(wvb_q8_kernel<16>, grid, dim3(256), 0, stream, a);
