@@ -120,9 +120,22 @@ __global__ __launch_bounds__(256) void wvb_q8_kernel(WvbArgs a) {
 
 // ---- several tokens (chunked prefill): wv_b and WKB as tiled products ----
 // The per-token kernels above re-read the head's weights and re-quantise its activations for every
-// few outputs of every token.  From Q8_GEMM_MIN_TOKENS tokens on a workgroup takes 32 tokens of one
-// head and quantises them once, into LDS.
-constexpr int Q8_GEMM_MIN_TOKENS = 16;
+// few outputs of every token.  Here a workgroup takes 32 tokens of one head and quantises them once,
+// into LDS.  Measured on the MI355X, 32 heads, per-token -> tiled kernel (us): wv_b 256 -> 128: 16
+// tokens 7.9 -> 9.9, 24 10.9 -> 10.2, 64 24.5 -> 10.5, 500 212 -> 20.4; 512 -> 128: 16 14.0 -> 18.7,
+// 24 19.8 -> 19.1, 64 48.8 -> 19.6.  WKB 64 -> 256: 32 tokens 3.0 -> 3.8, 64 4.4 -> 4.0, 500 22.3 ->
+// 7.6; 128 -> 512: 16 4.4 -> 4.1, 64 16.0 -> 5.1, 500 111 -> 14.0.  The per-token kernels' time goes
+// with their workgroups (or rows), the tiled ones' has a floor of one tile's latency, so the lines lie
+// at a number of workgroups (wv_b: 24 tokens x 32 heads x 16) and at a number of rows times their
+// length (WKB: 56 tokens x 32 heads x 256 rows x 64), and no tile is mostly empty below 8 tokens.
+constexpr int Q8_GEMM_MIN_TOKENS = 8;
+inline bool wvb_tiled(const WvbArgs & a) {
+    return a.nt >= Q8_GEMM_MIN_TOKENS && (int64_t)a.nt * a.n_head * ((a.d_out + 7) / 8) >= 24 * 32 * 16 &&
+           a.d_out <= 128 * 65535;          // its grid's y
+}
+inline bool wkb_q8_tiled(const WkbArgs & a) {
+    return a.nt >= Q8_GEMM_MIN_TOKENS && (int64_t)a.nt * a.n_head * ((a.d_v + 255) / 256) * a.d_n >= 56 * 32 * 64;
+}
 constexpr int GT = 32;                   // tokens per workgroup
 constexpr uint32_t Q_PAD = 16;           // LDS row padding: rows start on distinct banks
 
@@ -213,8 +226,8 @@ __device__ __forceinline__ void quant_tokens(const char * x, int64_t x_nbt, int 
 // element) computes with the same single rounding.  Its two blocks take positions j and j + 16, whose
 // sums are the butterfly's first step; the other steps are additions of accumulators in the
 // butterfly's order (16, 8, 4, 2, 1), so the result is the per-token kernel's bit for bit.
-// Bound: 2 x 16 NB MFMAs of 64 cycles per SIMD at two waves (NB = 8: 6.8 us for the 1,024 waves
-// of 512 tokens x 32 heads).
+// Bound: its MFMAs, 16 NB of 64 cycles per wave (NB = 8, 500 tokens x 32 heads: 2,048 waves, two per
+// SIMD, 6.8 us); 20.4 us there against 212 us for the per-token kernel.
 template <int NB>
 __global__ __launch_bounds__(256, NB <= 8 ? 2 : 1) void wvb_q8_gemm_kernel(WvbArgs a) {
     static_assert(NB % 2 == 0 && NB >= 4, "rows of an even number of blocks are 4-byte aligned");
@@ -286,7 +299,7 @@ __global__ __launch_bounds__(256, NB <= 8 ? 2 : 1) void wvb_q8_gemm_kernel(WvbAr
     }
 }
 
-// WKB over 32 tokens of one head, every output: wave w takes 32-column blocks w, w + 4, ...  The
+// WKB over 32 tokens of one head: wave w of column group z takes 32-column blocks 4 z + w, + 4 Z, ...  The
 // int32 dot of one Q8 block is one v_mfma_i32_32x32x32_i8 (exact), then acc = fma(wd * d16, sum,
 // acc) over the blocks in order, the per-token kernel's operations bit for bit.
 template <int NB>
@@ -307,7 +320,7 @@ __global__ __launch_bounds__(256) void wkb_q8_gemm_kernel(WkbArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) xs[b][i] = *reinterpret_cast<const f32x4 *>(&xd[b][8 * i + 4 * kh]);
     }
-    for (int c0 = 32 * w; c0 < a.d_v; c0 += 128) {
+    for (int c0 = 128 * blockIdx.z + 32 * w; c0 < a.d_v; c0 += 128 * gridDim.z) {
         const int c = c0 + r;
         const uint8_t * wrow = a.wq + ((size_t)h * a.d_v + min(c, a.d_v - 1)) * (NB * 34);
         u32x4 qw[NB];
@@ -471,8 +484,10 @@ __global__ __launch_bounds__(1024) void kvwrite_tail_kernel(KvWriteArgs a) {
 }  // namespace
 
 hipError_t launch_wkb_q8(const WkbArgs & a, hipStream_t stream) {
-    if (a.nt >= Q8_GEMM_MIN_TOKENS) {
-        const dim3 grid(a.n_head, (a.nt + GT - 1) / GT);
+    if (wkb_q8_tiled(a)) {
+        // few workgroups: the columns are split over them too
+        const int tb = (a.nt + GT - 1) / GT;
+        const dim3 grid(a.n_head, tb, a.n_head * tb < 256 && a.d_v <= 128 * 65535 ? (a.d_v + 127) / 128 : 1);
         if (a.d_n == 64) hipLaunchKernelGGL(wkb_q8_gemm_kernel<2>, grid, dim3(256), 0, stream, a);
         else if (a.d_n == 128) hipLaunchKernelGGL(wkb_q8_gemm_kernel<4>, grid, dim3(256), 0, stream, a);
         else return hipErrorInvalidValue;
@@ -486,7 +501,7 @@ hipError_t launch_wkb_q8(const WkbArgs & a, hipStream_t stream) {
 }
 
 hipError_t launch_wvb_q8(const WvbArgs & a, hipStream_t stream) {
-    if (a.nt >= Q8_GEMM_MIN_TOKENS) {
+    if (wvb_tiled(a)) {
         const dim3 grid((a.nt + GT - 1) / GT, (a.d_out + 127) / 128, a.n_head);
         if (a.d_in == 256) hipLaunchKernelGGL(wvb_q8_gemm_kernel<8>, grid, dim3(256), 0, stream, a);
         else if (a.d_in == 512) hipLaunchKernelGGL(wvb_q8_gemm_kernel<16>, grid, dim3(256), 0, stream, a);
