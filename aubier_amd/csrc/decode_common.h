@@ -82,6 +82,24 @@ struct PvAddr {
     }
 };
 
+// The same for P as the pair Q.K^T below leaves it (prefill): the MFMA's k index 8 hi + e of a slice
+// (hi = lane >> 5) stands for key 4 hi + (e & 3) + 8 (e >> 2), so group g reads rows 4 (g >> 1) .. +3,
+// then + 8.  The eight rows of a read fall on every bank twice (512 bytes over 64 banks: no conflict;
+// rows 0 .. 3 and 8 .. 11 above share banks two by two).
+struct PairPvAddr {
+    int lo;                                  // tile 0 (chunks 0 .. 3); the second read is 1 KB on (row + 8)
+    __device__ __forceinline__ explicit PairPvAddr(int lane) {
+        const int g = lane >> 4, j16 = lane & 15;
+        lo = slot_byte(4 * (g >> 1) + (j16 >> 2), 2 * (g & 1) + ((j16 & 3) >> 1)) + 8 * (j16 & 1);
+    }
+    __device__ __forceinline__ half8 load(const char * sb, int i) const {
+        const char * p = sb + (lo ^ (64 * (i & 1))) + 2048 * (i >> 1);
+        const half4 l4 = lds_read_tr16(reinterpret_cast<const half_t *>(p));
+        const half4 h4 = lds_read_tr16(reinterpret_cast<const half_t *>(p + 1024));
+        return half8{l4[0], l4[1], l4[2], l4[3], h4[0], h4[1], h4[2], h4[3]};
+    }
+};
+
 struct SliceDma { i32x4 krs, mrs; uint32_t sb; };
 
 // The wave's view of its split: tile range, DMA of its slice of tile k into stage s.
@@ -198,17 +216,44 @@ __device__ __forceinline__ uint32_t live_rows_of_wave(const DecodeArgs & a, int 
     return bits;
 }
 
-// Whether token t has a live key (mask > -inf, key < n_kv) in the split's tiles: the mask row
-// read over the split's range (cached loads, one key per lane per step), OR-ed over the wavefront.
-// Every wave of the workgroup computes the same answer.  Without a mask every key below n_kv is live.
-template <int DK>
-__device__ __forceinline__ bool split_live(const DecodeArgs & a, const SliceStream<DK> & ss, int t, int lane) {
-    const int k0 = ss.t0 * TK, k1 = min((ss.t0 + ss.n_my) * TK, a.n_kv);
-    if (a.mask == nullptr) return k0 < k1;
-    const float * row = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.mask) + (size_t)t * a.mask_nb1);
-    bool live = false;
-    for (int k = k0 + lane; k < k1; k += 64) live |= row[k] != -INFINITY;
-    return __builtin_amdgcn_ballot_w64(live) != 0;
+// The first and last live key (mask > -inf) of the mask row in [k0, k1) (first > last: none; without a
+// mask every key is live), found from the two ends in rounds of 1,024 keys, every load of a round
+// issued before its first compare: the indices are clamped rather than the loads guarded (a guarded
+// load is a branch and a wait of its own, the memory latency per 64 keys: 20 us per launch at 1,000
+// keys).  The whole wavefront computes one answer.
+__device__ __forceinline__ void live_keys(const float * row, int k0, int k1, int lane, int & first, int & last) {
+    last = k0 - 1;
+    if (row == nullptr) {
+        first = k0;
+        last = max(k0, k1) - 1;
+        return;
+    }
+    k1 = max(k0, k1);
+    first = k1;
+    constexpr int N = 16;
+    auto round = [&](int kb, bool fwd) {       // keys kb .. kb + 64 N - 1, those in [k0, k1)
+        float v[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] = row[min(max(kb + 64 * j + lane, k0), k1 - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+        int f = -1, l = -1;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int k = kb + 64 * j + lane;
+            const uint64_t b = __builtin_amdgcn_ballot_w64(k >= k0 && k < k1 && v[j] != -INFINITY);
+            f = (b != 0 && f < 0) ? kb + 64 * j + __builtin_ctzll(b) : f;
+            l = b != 0 ? kb + 64 * j + 63 - __builtin_clzll(b) : l;
+        }
+        return fwd ? f : l;
+    };
+    for (int kb = k0; kb < k1 && first == k1; kb += 64 * N) {
+        const int f = round(kb, true);
+        if (f >= 0) first = f;
+    }
+    for (int ke = k1; ke > first && last < first; ke -= 64 * N) {
+        const int l = round(ke - 64 * N, false);
+        if (l >= 0) last = l;
+    }
 }
 
 // The (m, l) pairs of a split with no live key: m = -inf, l = 0 for the record's 32 heads; its o
@@ -293,24 +338,9 @@ __device__ __forceinline__ void stage_q(const DecodeArgs & a, const SliceStream<
     __syncthreads();                         // the q staging in stage 1 is free again
 }
 
-// acc += a . b (v_mfma_f32_16x16x32_f16; first: acc = a . b).  VACC keeps acc in VGPRs through
-// inline asm: in the kernels whose output accumulators fill all 256 AGPRs the compiler selects the
-// AGPR form for every MFMA and would move an output tile out to VGPRs and back around each Q.K^T
-// (48 v_accvgpr moves per slice).  Inline asm is outside the compiler's hazard tracking, so the
-// caller covers the MFMA -> VALU read distance (vacc_settle) before it reads the result.
-template <bool VACC>
+// acc += a . b (v_mfma_f32_16x16x32_f16; first: acc = a . b)
 __device__ __forceinline__ void mfma16(f32x4 & acc, const half8 & a, const half8 & b, bool first) {
-    if constexpr (VACC) {
-        if (first) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
-        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
-    } else {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc, 0, 0, 0);
-    }
-}
-// 24 wait states after the last MFMA writing acc0..acc3, ahead of any VALU read of them (the
-// operands tie the reads to this point)
-__device__ __forceinline__ void vacc_settle(f32x4 & acc0, f32x4 & acc1, f32x4 & acc2, f32x4 & acc3) {
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(acc0), "+v"(acc1), "+v"(acc2), "+v"(acc3));
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, first ? f32x4{0.f, 0.f, 0.f, 0.f} : acc, 0, 0, 0);
 }
 
 // S^T = K . Q^T for the wave's 16 keys of the slice at sb (C rows = keys 4 g + r, C cols = heads
@@ -321,12 +351,10 @@ __device__ __forceinline__ void vacc_settle(f32x4 & acc0, f32x4 & acc1, f32x4 & 
 // With DMA, the next slice's DMA (dn, streaming cache policy) is spread over the steps.  Operand
 // reads run QPF steps ahead of their MFMAs; the scheduling barriers keep the compiler from sinking
 // them back next to their use.  Two accumulator chains per head tile (even / odd steps) keep
-// consecutive MFMAs independent.  Returns with the slice's mask slot landed.  WAIT = false: the
-// slice is known to be in LDS already (no DMA accounting, no next-slice DMA).
-template <int DK, bool DMA, bool WAIT = true>
+// consecutive MFMAs independent.  Returns with the slice's mask slot landed.
+template <int DK, bool DMA>
 __device__ __forceinline__ void qk_slice(const SliceStream<DK> & ss, const SliceDma & dn, const char * sb, int lane,
                                          const half8 (&qreg)[2][SliceGeom<DK>::QSTEPS], f32x4 & s0, f32x4 & s1) {
-    static_assert(WAIT || !DMA, "a slice already in LDS comes with no DMA to spread");
     using G = SliceGeom<DK>;
     constexpr int QPF = 4;
     const int g = lane >> 4, j16 = lane & 15;
@@ -336,7 +364,7 @@ __device__ __forceinline__ void qk_slice(const SliceStream<DK> & ss, const Slice
     const int a0 = slot_byte(j16, g);
     auto arow = [&](int st) { return reinterpret_cast<const half8 *>(sb + (a0 ^ (64 * (st & 1))) + 2048 * (st >> 1)); };
     half8 abuf[QPF];
-    if constexpr (WAIT) wait_vm<G::DMA_N + 1 - QPF>();      // blocks 0 .. QPF - 1
+    wait_vm<G::DMA_N + 1 - QPF>();      // blocks 0 .. QPF - 1
 #pragma unroll
     for (int s = 0; s < QPF; ++s) abuf[s] = *arow(s);
 #pragma unroll
@@ -346,15 +374,15 @@ __device__ __forceinline__ void qk_slice(const SliceStream<DK> & ss, const Slice
             // blocks 0 .. 2 ((s + QPF) >> 1) + 1 landed; s instructions of the next slice issued
             const int later = G::DMA_N - 1 - 2 * ((s + QPF) >> 1);
             if constexpr (DMA) wait_vm_le(later + s);
-            else if constexpr (WAIT) wait_vm_le(later);
+            else wait_vm_le(later);
             abuf[s % QPF] = *arow(s + QPF);
         }
         if (s & 1) {
-            mfma16<false>(acc2, av, qreg[0][s], s == 1);
-            mfma16<false>(acc3, av, qreg[1][s], s == 1);
+            mfma16(acc2, av, qreg[0][s], s == 1);
+            mfma16(acc3, av, qreg[1][s], s == 1);
         } else {
-            mfma16<false>(acc0, av, qreg[0][s], s == 0);
-            mfma16<false>(acc1, av, qreg[1][s], s == 0);
+            mfma16(acc0, av, qreg[0][s], s == 0);
+            mfma16(acc1, av, qreg[1][s], s == 0);
         }
         if constexpr (DMA) ss.put(dn, s);
         __builtin_amdgcn_sched_barrier(0);
@@ -362,51 +390,51 @@ __device__ __forceinline__ void qk_slice(const SliceStream<DK> & ss, const Slice
     if constexpr (DMA) {
         ss.put(dn, G::DMA_N);
         wait_vm<G::DMA_N + 1>();             // the mask slot (the next slice's DMA_N + 1 may be in flight)
-    } else if constexpr (WAIT) {
+    } else {
         wait_vm<0>();
     }
     s0 = acc0 + acc2;
     s1 = acc1 + acc3;
 }
 
-// Q.K^T of a slice already in LDS (no DMA accounting; the prefill's tiles land before a barrier),
-// accumulators in VGPRs.  Operand block st of the wave's rows is read QPF_LANDED steps ahead; the
+// Q.K^T of two slices already in LDS (no DMA accounting; the prefill's tiles land before a barrier):
+// S^T = K . Q^T for 32 keys (slices at sb and sb + STAGE) x 32 heads on v_mfma_f32_32x32x16_f16, the
+// accumulator in VGPRs: element r is key 8 (r / 4) + 4 (lane >> 5) + (r & 3) of head lane & 31, so a
+// lane holds one head's scores and its P is P.V's operand without a lane exchange.  The MFMAs are
+// inline asm: the output tiles fill the AGPRs, and the compiler, which selects the AGPR form for every
+// MFMA of such a kernel, would move one of them out and back around each Q.K^T.  qf[st] = head
+// lane & 31, d = 16 st + 8 (lane >> 5) .. +7.  Operand step st is read QPF_LANDED steps ahead; the
 // first QPF_LANDED come in `abuf` (qk_operands, which the caller may issue early so that their LDS
-// latency passes under other work).  hook(s) runs after step s's MFMAs: the caller's DMA of the
+// latency passes under other work).  hook(st) runs after step st's MFMA: the caller's DMA of the
 // next tile, spread over the steps.
 constexpr int QPF_LANDED = 4;
+// step st (chunks 2 st, 2 st + 1) of this lane's key: row lane & 15 of slice (lane >> 4) & 1
+template <int DK>
+__device__ __forceinline__ half8 qk_pair_operand(const char * sb, int lane, int st) {
+    const int c0 = slot_byte(lane & 15, lane >> 5) + SliceGeom<DK>::STAGE * ((lane >> 4) & 1);
+    return *reinterpret_cast<const half8 *>(sb + (c0 ^ (32 * (st & 3))) + 2048 * (st >> 2));
+}
 template <int DK>
 __device__ __forceinline__ void qk_operands(const char * sb, int lane, half8 (&abuf)[QPF_LANDED]) {
-    const int a0 = slot_byte(lane & 15, lane >> 4);
 #pragma unroll
-    for (int st = 0; st < QPF_LANDED; ++st)
-        abuf[st] = *reinterpret_cast<const half8 *>(sb + (a0 ^ (64 * (st & 1))) + 2048 * (st >> 1));
+    for (int st = 0; st < QPF_LANDED; ++st) abuf[st] = qk_pair_operand<DK>(sb, lane, st);
 }
 template <int DK, typename H>
-__device__ __forceinline__ void qk_slice_landed(const char * sb, int lane, const half8 (&qreg)[2][SliceGeom<DK>::QSTEPS],
-                                                half8 (&abuf)[QPF_LANDED], f32x4 & s0, f32x4 & s1, H && hook) {
-    using G = SliceGeom<DK>;
+__device__ __forceinline__ void qk_pair_landed(const char * sb, int lane, const half8 (&qf)[DK / 16],
+                                               half8 (&abuf)[QPF_LANDED], f32x16 & s, H && hook) {
     constexpr int QPF = QPF_LANDED;
-    const int a0 = slot_byte(lane & 15, lane >> 4);
-    auto arow = [&](int st) { return reinterpret_cast<const half8 *>(sb + (a0 ^ (64 * (st & 1))) + 2048 * (st >> 1)); };
-    f32x4 acc0, acc1, acc2, acc3;
 #pragma unroll
-    for (int s = 0; s < G::QSTEPS; ++s) {
-        const half8 av = abuf[s % QPF];
-        if (s + QPF < G::QSTEPS) abuf[s % QPF] = *arow(s + QPF);
-        if (s & 1) {
-            mfma16<true>(acc2, av, qreg[0][s], s == 1);
-            mfma16<true>(acc3, av, qreg[1][s], s == 1);
-        } else {
-            mfma16<true>(acc0, av, qreg[0][s], s == 0);
-            mfma16<true>(acc1, av, qreg[1][s], s == 0);
-        }
-        hook(s);
+    for (int st = 0; st < DK / 16; ++st) {
+        const half8 av = abuf[st % QPF];
+        if (st + QPF < DK / 16) abuf[st % QPF] = qk_pair_operand<DK>(sb, lane, st + QPF);
+        if (st == 0) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(s) : "v"(av), "v"(qf[st]));
+        else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(s) : "v"(av), "v"(qf[st]));
+        hook(st);
         __builtin_amdgcn_sched_barrier(0);
     }
-    vacc_settle(acc0, acc1, acc2, acc3);
-    s0 = acc0 + acc2;
-    s1 = acc1 + acc3;
+    // 24 wait states after the last MFMA, ahead of any VALU read of s (inline asm is outside the
+    // compiler's hazard tracking)
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(s));
 }
 
 // the mask values of keys 4 g .. 4 g + 3 of the slice at sb (its mask slot)
@@ -417,8 +445,7 @@ __device__ __forceinline__ f32x4 slice_mask(const char * sb, int lane) {
 
 // Scores in log2 units of keys kbase + 4 g + r for heads j16 (sc[0]) and 16 + j16 (sc[1]); masked,
 // padded and out-of-range keys are -inf.  mk = the mask values of those 4 keys (zeros without a
-// mask).  mx = the slice's max per head over its 16 keys (ACROSS), or over this lane's 4 keys.
-template <bool ACROSS = true>
+// mask).  mx = the slice's max per head over its 16 keys.
 __device__ __forceinline__ void slice_scores(const DecodeArgs & a, const f32x4 & mk, int kbase, int lane, const f32x4 & s0,
                                              const f32x4 & s1, float (&sc)[2][4], float (&mx)[2]) {
     const int g = lane >> 4;
@@ -434,17 +461,15 @@ __device__ __forceinline__ void slice_scores(const DecodeArgs & a, const f32x4 &
         mx[0] = fmaxf(mx[0], sc[0][r]);
         mx[1] = fmaxf(mx[1], sc[1][r]);
     }
-    if constexpr (ACROSS) {
 #pragma unroll
-        for (int n = 0; n < 2; ++n) mx[n] = rows4_max(mx[n]);
-    }
+    for (int n = 0; n < 2; ++n) mx[n] = rows4_max(mx[n]);
 }
 
 // Whether a head's lazily moved reference max m (M_NONE before its first live key) must move for
 // scores whose max is x: x exceeds m by more than 2^LAZY (any live key, while m = M_NONE).  A
-// head's slice max exceeds the bound iff one of its four lanes' own maxima does, so the kernels
-// test the lanes' own maxima first and take the cross-lane max only on the (rare) path where some
-// reference moves.
+// head's max exceeds the bound iff one of its lanes' own maxima does, so the prefill kernel tests the
+// lanes' own maxima first and takes the cross-lane max only on the (rare) path where some reference
+// moves.
 __device__ __forceinline__ bool ref_moves(float m, float x) { return x > m + LAZY; }
 
 // ---------------------------------------------------------------- the decode kernels

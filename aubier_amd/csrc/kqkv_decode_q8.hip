@@ -157,11 +157,11 @@ __device__ __forceinline__ void qk_slice_q8(const char * src, char * dst, int la
         if (s + PF < G::QSTEPS) rd(s + PF);
         if (32 * s < DV) *reinterpret_cast<half8 *>(dst + (a0 ^ (64 * (s & 1))) + 2048 * (s >> 1)) = av;
         if (s & 1) {
-            mfma16<false>(acc2, av, qreg[0][s], s == 1);
-            mfma16<false>(acc3, av, qreg[1][s], s == 1);
+            mfma16(acc2, av, qreg[0][s], s == 1);
+            mfma16(acc3, av, qreg[1][s], s == 1);
         } else {
-            mfma16<false>(acc0, av, qreg[0][s], s == 0);
-            mfma16<false>(acc1, av, qreg[1][s], s == 0);
+            mfma16(acc0, av, qreg[0][s], s == 0);
+            mfma16(acc1, av, qreg[1][s], s == 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     }

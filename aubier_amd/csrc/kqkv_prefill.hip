@@ -12,19 +12,24 @@
 //     LDS ring (decode_common.h layout, cached DMA: the cache is re-read by every token group and
 //     stays in L2 / MALL) plus its own token's 64 mask values, and then every wave runs all four
 //     slices -- 4 tokens x 32 heads share each K / V byte read from LDS.  One workgroup barrier
-//     per tile; the next tile's DMA goes out one instruction per even Q.K^T step of the first two
-//     slices.
-//   * Per slice: S^T = K . Q^T (16 keys x 32 heads, v_mfma_f32_16x16x32_f16, accumulators in
-//     VGPRs: the output tiles fill the AGPRs), scores with the token's mask, a lazily moved
-//     reference max (P = exp2(s - m) <= 2^15; the move test on each lane's own maxima), P^T for P.V
-//     by two v_permlane16_swap, o^T += V^T . P^T (v_mfma_f32_32x32x16_f16, V^T by
-//     ds_read_b64_tr_b16).  l is summed from the same f16 P values.  q enters as f16, where
-//     ggml-cpu's mul_mat rounds it; P enters as f16 too, but UNNORMALISED (exp2 of the score minus
-//     the lazy reference max, <= 2^15), where ggml-cpu rounds the normalised softmax output -- at
-//     long context the latter is subnormal in f16, so the two differ by more than one rounding
-//     (this kernel is the closer of the two to exact arithmetic).  The next slice's first Q.K^T
-//     operands and mask values are read
-//     during P.V, the first V^T operands during the softmax.
+//     per tile; the next tile's DMA goes out one instruction per fourth Q.K^T step.
+//   * Per pair of slices (32 keys): S^T = K . Q^T (32 keys x 32 heads, v_mfma_f32_32x32x16_f16, the
+//     accumulator in VGPRs: the output tiles fill the AGPRs), scores with the token's mask, a lazily
+//     moved reference max (P = exp2(s - m) <= 2^15; the move test on each lane's own maximum), then
+//     o^T += V^T . P^T (v_mfma_f32_32x32x16_f16, V^T by ds_read_b64_tr_b16).  A lane of S^T holds 16
+//     scores of one head, which are P.V's operand as they lie (the k order of that MFMA is free as long
+//     as V^T is read in the same one): no lane exchange, and conflict-free transpose reads.  Slice 1's
+//     exponentials and the sums of P run between slice 0's P.V MFMAs.  l is summed from the same f16
+//     P values.  q enters as f16, where ggml-cpu's mul_mat rounds it; P enters as f16 too, but
+//     UNNORMALISED (exp2 of the score minus the lazy reference max, <= 2^15), where ggml-cpu rounds
+//     the normalised softmax output -- at long context the latter is subnormal in f16, so the two
+//     differ by more than one rounding (this kernel is the closer of the two to exact arithmetic).
+//   * The loop runs over the tiles that hold a live key of the workgroup's tokens (live_keys).
+// Measured on the MI355X, D_k 576, 1,024 tokens x 32 heads in one split, no mask: 4,096 keys 262 us =
+// 1.11 PFLOP/s (287 us with one slice at a time and serial reads of the mask row), 64 keys 26 us
+// (28).  A tile takes 2.9 us of its 1.8 us of MFMA with few workgroups or with all-zero operands and
+// 3.9 us with ordinary ones on all 256 CUs, where the clock drops: at full load the kernel is bound
+// by power, at a rate near the card's large f16 matrix product (1.17 PFLOP/s).  At 320: 157 us (197).
 //
 // Grid = (n_split, ceil(H/32), ceil(nt/4)), 256 threads.  Output as the decode kernels: partial
 // blocks [group][token][split] (mla_kernels.h) for the merge, or o/l in f32 to dst with one split.
@@ -52,15 +57,15 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_prefill_f16_kernel(DecodeArgs a)
     using G = SliceGeom<DK>;
     using C = PrefillCfg<DK, DV>;
     __shared__ __attribute__((aligned(16))) char ring[G::RING];          // [stage][wave] K rows + mask
+    __shared__ int live_of[NWAVE][2];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sp = blockIdx.x;
     const int hg0 = blockIdx.y * HG;
-    const int g = lane >> 4;
-    const int j16 = lane & 15;
-    const int t_w = blockIdx.z * NWAVE + w;          // this wave's token
+    // this wave's token; the last token groups, which see the most keys under a causal mask, start first
+    const int t_w = ((int)gridDim.z - 1 - (int)blockIdx.z) * NWAVE + w;
     const bool token_live = t_w < a.nt;
     const int t = min(t_w, a.nt - 1);                // (a wave past the last token mirrors it, unused)
 
@@ -77,185 +82,203 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_prefill_f16_kernel(DecodeArgs a)
         d.mrs = make_rsrc(ss.mrow + tile * TK, (ss.has_mask && mleft > 0) ? (uint32_t)mleft * 4u : 0u);
         return d;
     };
-    // Rows over per-sequence regions (batch-of-N decode): a wave whose token has no live key in this
-    // split still streams its slices for the others but computes nothing; a workgroup with no live
-    // token records empty splits and leaves before any DMA.  (One split writes dst directly: every
-    // row is computed.)
-    const bool live_w = token_live && (a.dst != nullptr || split_live<DK>(a, ss, t, lane));
-    if (!__syncthreads_or(live_w)) {
-        if (token_live && a.dst == nullptr) write_empty_pairs(a, blockIdx.y, t, sp, DV, lane);
+    // The tiles of the split that hold a live key (mask > -inf) of this wave's token, [ka_w, kz_w), and of
+    // any of the workgroup's, [ka, kz): the loop runs over the latter (a causal chunk's first tokens see
+    // few of the window's tiles; rows over per-sequence regions one run of them), and a wave computes
+    // only in its own.  A workgroup with no live key records empty splits and leaves before any DMA.
+    int first, last;
+    live_keys(ss.has_mask ? ss.mrow : nullptr, ss.t0 * TK, token_live ? min((ss.t0 + n_my) * TK, a.n_kv) : 0, lane, first, last);
+    const bool live_w = first <= last;
+    const int ka_w = live_w ? first / TK - ss.t0 : 0, kz_w = live_w ? last / TK - ss.t0 + 1 : 0;
+    if (lane == 0) {
+        live_of[w][0] = live_w ? ka_w : n_my;
+        live_of[w][1] = kz_w;
+    }
+    __syncthreads();
+    const int ka = min(min(live_of[0][0], live_of[1][0]), min(live_of[2][0], live_of[3][0]));
+    const int kz = max(max(live_of[0][1], live_of[1][1]), max(live_of[2][1], live_of[3][1]));
+    if (ka >= kz && a.dst == nullptr) {
+        if (token_live) write_empty_pairs(a, blockIdx.y, t, sp, DV, lane);
         return;
     }
     {
-        const SliceDma d0 = plan(0, 0);
+        const SliceDma d0 = plan(ka & 1, ka);
 #pragma unroll
         for (int i = 0; i <= G::DMA_N; ++i) ss.template put<false>(d0, i);
     }
 
-    // ---- q fragments of this wave's token: qreg[n][s] = head 16 n + j16, d = 32 s + 8 g .. +7 ----
-    half8 qreg[2][G::QSTEPS];
+    // ---- q fragments of this wave's token: qf[st] = head lane & 31, d = 16 st + 8 (lane >> 5) .. +7 ----
+    // Read in batches of QB fragments, each batch's loads issued before the one ahead of it is
+    // converted: a batch at a time, every batch paid the memory latency.
+    const int hl = lane & 31, hi = lane >> 5;
+    half8 qf[DK / 16];
     {
-        constexpr int QB = G::QSTEPS % 6 == 0 ? 6 : (G::QSTEPS % 5 == 0 ? 5 : 2);
+        constexpr int QB = DK / 16 % 6 == 0 ? 6 : 5;
+        constexpr int NBT = DK / 16 / QB;
+        static_assert(NBT * QB == DK / 16, "whole batches");
+        const bool hv = hg0 + hl < a.n_head;
+        const char * row = reinterpret_cast<const char *>(a.q) + (size_t)t * a.q_nb2 +
+                           (size_t)min(hg0 + hl, a.n_head - 1) * a.q_nb1 + 32 * hi;
+        f32x4 x[2][QB][2];
+        auto load = [&](int i, f32x4 (&xb)[QB][2]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
-            const int h = hg0 + 16 * n + j16;
-            const bool hv = h < a.n_head;
-            const char * row = reinterpret_cast<const char *>(a.q) + (size_t)t * a.q_nb2 + (size_t)min(h, a.n_head - 1) * a.q_nb1;
-#pragma unroll
-            for (int s0 = 0; s0 < G::QSTEPS; s0 += QB) {
-                f32x4 x[QB][2];
-#pragma unroll
-                for (int b = 0; b < QB; ++b) {
-                    x[b][0] = *reinterpret_cast<const f32x4 *>(row + 4 * (32 * (s0 + b) + 8 * g));
-                    x[b][1] = *reinterpret_cast<const f32x4 *>(row + 4 * (32 * (s0 + b) + 8 * g + 4));
-                }
-#pragma unroll
-                for (int b = 0; b < QB; ++b) {
-                    half8 hq = {to_half(x[b][0][0]), to_half(x[b][0][1]), to_half(x[b][0][2]), to_half(x[b][0][3]),
-                                to_half(x[b][1][0]), to_half(x[b][1][1]), to_half(x[b][1][2]), to_half(x[b][1][3])};
-                    if (!hv) hq = half8{0, 0, 0, 0, 0, 0, 0, 0};
-                    asm volatile("" : "+v"(hq));     // keep the f16 fragment (not the f32 values) live
-                    qreg[n][s0 + b] = hq;
-                }
+            for (int b = 0; b < QB; ++b) {
+                xb[b][0] = *reinterpret_cast<const f32x4 *>(row + 64 * (QB * i + b));
+                xb[b][1] = *reinterpret_cast<const f32x4 *>(row + 64 * (QB * i + b) + 16);
             }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        load(0, x[0]);
+#pragma unroll
+        for (int i = 0; i < NBT; ++i) {
+            if (i + 1 < NBT) load(i + 1, x[(i + 1) & 1]);
+#pragma unroll
+            for (int b = 0; b < QB; ++b) {
+                const f32x4 (&y)[2] = x[i & 1][b];
+                half8 hq = {to_half(y[0][0]), to_half(y[0][1]), to_half(y[0][2]), to_half(y[0][3]),
+                            to_half(y[1][0]), to_half(y[1][1]), to_half(y[1][2]), to_half(y[1][3])};
+                if (!hv) hq = half8{0, 0, 0, 0, 0, 0, 0, 0};
+                asm volatile("" : "+v"(hq));         // keep the f16 fragment (not the f32 values) live
+                qf[QB * i + b] = hq;
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 
     // ---- per-wave state ----
-    float m_run[2] = {M_NONE, M_NONE};       // heads 16 n + j16, log2 units
-    float l_acc = 0.0f;                      // head lane & 31, keys 8 (lane >> 5) .. +7 of each slice
-    f32x16 o[C::NB];                         // o^T tile i: C row = column 32 i + 8 (r / 4) + 4 (lane >> 5) + (r & 3), C col = head lane & 31
+    float m_run = M_NONE;                    // head hl, log2 units
+    float l_acc = 0.0f;                      // head hl, this lane's half of the keys
+    f32x16 o[C::NB];                         // o^T tile i: C row = column 32 i + 8 (r / 4) + 4 hi + (r & 3), C col = head hl
 #pragma unroll
     for (int i = 0; i < C::NB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[i][r] = 0.0f;
-    const PvAddr pv(lane);
-    const int own_h = (lane >> 4) & 1;
+    const PairPvAddr pv(lane);
 
-    for (int k = 0; k < n_my; ++k) {
+    for (int k = ka; k < kz; ++k) {
         wait_vm<0>();                        // this wave's slot of tile k (and its mask row) has landed
         __syncthreads();                     // all four have; every wave is done with tile k - 1
-        const bool pf = k + 1 < n_my;
+        const bool pf = k + 1 < kz;
         const SliceDma dn = plan((k + 1) & 1, k + 1);
         const int par = k & 1;
         const int key_t = (ss.t0 + k) * TK;
         const char * mkb = ring + ss.stage_off(par, w) + G::ROWS_BYTES;    // this token's mask, 64 keys
-        if (!live_w) {                       // only this wave's slice of the next tile
+        if (k < ka_w || k >= kz_w) {         // only this wave's slice of the next tile
             if (pf) {
 #pragma unroll
                 for (int i = 0; i <= G::DMA_N; ++i) ss.template put<false>(dn, i);
             }
             continue;
         }
-        // slice 0's first Q.K^T operands and mask values (later slices': during the P.V before)
+        // the first pair's first Q.K^T operands (the second's: during the P.V before)
         half8 abuf[QPF_LANDED];
         qk_operands<DK>(ring + ss.stage_off(par, 0), lane, abuf);
-        f32x4 mk_next = *reinterpret_cast<const f32x4 *>(mkb + 16 * g);
 #pragma unroll 1
-        for (int ks = 0; ks < NWAVE; ++ks) {
-            const char * sb = ring + ss.stage_off(par, ks);
-            const f32x4 mk = mk_next;
-            f32x4 s0, s1;
-            // tile k + 1's DMA, one instruction per even Q.K^T step of slices 0 and 1 (row blocks
-            // DMA_N / 2 * ks + s / 2) and the mask slot after slice 1's last step: the CU's 76 KB of
-            // DMA per tile, issued within one slice, held the issuing waves ~450 cycles
-            if (pf && ks < 2) {
-                qk_slice_landed<DK>(sb, lane, qreg, abuf, s0, s1, [&](int st) {
+        for (int kp = 0; kp < NWAVE / 2; ++kp) {
+            const char * sb = ring + ss.stage_off(par, 2 * kp);
+            f32x16 s;
+            // tile k + 1's DMA, one instruction per fourth Q.K^T step (row blocks DMA_N / 2 * kp + st / 4)
+            // and the mask slot after the second pair's last step: the CU's 76 KB of DMA per tile,
+            // issued at once, held the issuing waves ~450 cycles
+            if (pf) {
+                qk_pair_landed<DK>(sb, lane, qf, abuf, s, [&](int st) {
                     constexpr int HALF = G::DMA_N / 2;
-                    static_assert(G::DMA_N % 2 == 0 && G::QSTEPS == G::DMA_N, "two slices of row blocks");
-                    if ((st & 1) == 0) ss.template put<false>(dn, HALF * ks + st / 2);
-                    else if (st == G::QSTEPS - 1 && ks == 1) ss.template put<false>(dn, G::DMA_N);
+                    static_assert(G::DMA_N % 2 == 0 && DK / 16 == 2 * G::DMA_N, "two pairs of slices of row blocks");
+                    if ((st & 3) == 0) ss.template put<false>(dn, HALF * kp + st / 4);
+                    else if (st == DK / 16 - 1 && kp == 1) ss.template put<false>(dn, G::DMA_N);
                 });
             } else {
-                qk_slice_landed<DK>(sb, lane, qreg, abuf, s0, s1, [](int) {});
+                qk_pair_landed<DK>(sb, lane, qf, abuf, s, [](int) {});
             }
-            // the first V^T operands of P.V, read ahead so that their latency passes under the softmax
+            // the pair's mask values of this lane's keys and the first V^T operands of P.V, read ahead so
+            // that their latency passes under the scores and the softmax
+            f32x4 mk[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mk[j] = *reinterpret_cast<const f32x4 *>(mkb + 4 * (32 * kp + 8 * j + 4 * hi));
             constexpr int VPF = 3;
             half8 vb[VPF];
 #pragma unroll
             for (int i = 0; i < VPF; ++i) vb[i] = pv.load(sb, i);
             __builtin_amdgcn_sched_barrier(0);
-            float sc[2][4], mx[2];
-            slice_scores<false>(a, mk, key_t + WK * ks, lane, s0, s1, sc, mx);     // this lane's maxima
-            if (__builtin_amdgcn_ballot_w64(ref_moves(m_run[0], mx[0]) || ref_moves(m_run[1], mx[1])) != 0) {
-                // rare: move the reference to the head's slice max, rescale
-                float al[2];
-                bool mv[2];
+            // scores in log2 units; a key past n_kv (its K row and mask read as zeros) takes -inf
+            const int key0 = key_t + 32 * kp + 4 * hi;
+            if (key_t + TK > a.n_kv) {
 #pragma unroll
-                for (int n = 0; n < 2; ++n) {
-                    mx[n] = rows4_max(mx[n]);
-                    mv[n] = ref_moves(m_run[n], mx[n]);
-                    al[n] = !mv[n] ? 1.0f : exp2_fast(m_run[n] - mx[n]);     // 0 from M_NONE
-                    m_run[n] = mv[n] ? mx[n] : m_run[n];
-                }
-                const float a_own = al[own_h];
-                l_acc *= a_own;
-                // in place on the accumulator registers (kept in AGPRs); the s_nops cover the
-                // MFMA -> VALU read distance
-                asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-#pragma unroll
-                for (int i = 0; i < C::NB; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        float tmp;
-                        asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
-                                     : "+a"(o[i][r]), "=&v"(tmp) : "v"(a_own));
-                    }
-                asm volatile("s_nop 7" ::: "memory");
+                for (int r = 0; r < 16; ++r)
+                    if (key0 + 8 * (r >> 2) + (r & 3) >= a.n_kv) mk[r >> 2][r & 3] = -INFINITY;
             }
-            // P^T operand: Q.K^T's C layout (lane: keys 4 g .. +3 of heads j16 and 16 + j16) into
-            // P.V's B layout (lane: keys 8 (lane >> 5) .. +7 of head lane & 31), one
-            // v_permlane16_swap per pair of f16 values
-            uint32_t px[2], py[2];
+            float mx = -INFINITY;
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float x0 = exp2_fast(sc[0][2 * e] - m_run[0]);
-                const float x1 = exp2_fast(sc[0][2 * e + 1] - m_run[0]);
-                const float y0 = exp2_fast(sc[1][2 * e] - m_run[1]);
-                const float y1 = exp2_fast(sc[1][2 * e + 1] - m_run[1]);
-                px[e] = __builtin_bit_cast(uint32_t, half2{to_half(x0), to_half(x1)});
-                py[e] = __builtin_bit_cast(uint32_t, half2{to_half(y0), to_half(y1)});
-                const auto sw = __builtin_amdgcn_permlane16_swap(px[e], py[e], false, false);
-                px[e] = sw[0];
-                py[e] = sw[1];
+            for (int r = 0; r < 16; ++r) {
+                s[r] = s[r] * a.scale_log2 + mk[r >> 2][r & 3] * LOG2E;
+                mx = fmaxf(mx, s[r]);
             }
-            const half8 pt = __builtin_bit_cast(half8, u32x4{px[0], px[1], py[0], py[1]});
+            if (__builtin_amdgcn_ballot_w64(ref_moves(m_run, mx)) != 0) {
+                // rare: move the reference to the head's max over the pair, rescale
+                float lo, up;
+                halves_pair(mx, lo, up);
+                mx = fmaxf(lo, up);
+                const bool mv = ref_moves(m_run, mx);
+                // a head with no live key so far holds zeros: nothing to rescale
+                const bool scale = mv && m_run != M_NONE;
+                const float al = scale ? exp2_fast(m_run - mx) : 1.0f;
+                m_run = mv ? mx : m_run;
+                if (__builtin_amdgcn_ballot_w64(scale) != 0) {
+                    l_acc *= al;
+                    // in place on the accumulator registers (kept in AGPRs); the s_nops cover the
+                    // MFMA -> VALU read distance
+                    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) l_acc = __builtin_amdgcn_fdot2(half2{pt[e], pt[e + 1]}, ONE2, l_acc, false);
-            {
+                    for (int i = 0; i < C::NB; ++i)
 #pragma unroll
-                for (int i = 0; i < C::NB; ++i) {
-                    const half8 va = vb[i % VPF];
-                    if (i + VPF < C::NB) vb[i % VPF] = pv.load(sb, i + VPF);
-                    o[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt, o[i], 0, 0, 0);
-                    if (i == C::NB / 2 && ks + 1 < NWAVE) {     // the next slice's operands and mask
-                        qk_operands<DK>(ring + ss.stage_off(par, ks + 1), lane, abuf);
-                        mk_next = *reinterpret_cast<const f32x4 *>(mkb + 64 * (ks + 1) + 16 * g);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (int r = 0; r < 16; ++r) {
+                            float tmp;
+                            asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
+                                         : "+a"(o[i][r]), "=&v"(tmp) : "v"(al));
+                        }
+                    asm volatile("s_nop 7" ::: "memory");
                 }
+            }
+            // P^T operands of the two slices, P.V of the slices in turn; slice 1's exponentials and the sums
+            // of P run between slice 0's MFMAs (32 cycles each, which cover a few VALU instructions of
+            // the same wave)
+            half8 pt[2];
+            auto put_p = [&](int j, int e0) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = e0; e < e0 + 4; ++e) pt[j][e] = to_half(exp2_fast(s[8 * j + e] - m_run));
+            };
+            put_p(0, 0);
+            put_p(0, 4);
+#pragma unroll
+            for (int u = 0; u < 2 * C::NB; ++u) {
+                const half8 va = vb[u % VPF];
+                if (u + VPF < 2 * C::NB) vb[u % VPF] = pv.load(sb + G::STAGE * ((u + VPF) / C::NB), (u + VPF) % C::NB);
+                o[u % C::NB] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[u / C::NB], o[u % C::NB], 0, 0, 0);
+                if (u == 1) put_p(1, 0);
+                if (u == 3) put_p(1, 4);
+                if (u % C::NB < 4)
+                    l_acc = __builtin_amdgcn_fdot2(half2{pt[u / C::NB][2 * (u % C::NB)], pt[u / C::NB][2 * (u % C::NB) + 1]}, ONE2, l_acc, false);
+                if (u == C::NB + C::NB / 2 && kp + 1 < NWAVE / 2)       // the next pair's operands
+                    qk_operands<DK>(ring + ss.stage_off(par, 2 * kp + 2), lane, abuf);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
     wait_vm<0>();
     __syncthreads();                         // the ring becomes the output staging
-#pragma unroll
-    for (int n = 0; n < 2; ++n) m_run[n] = (m_run[n] == M_NONE) ? -INFINITY : m_run[n];     // no live key: -inf
-
     int tid_e;
     asm volatile("v_mov_b32 %0, %1" : "=v"(tid_e) : "v"(tid));
     const int lane_e = tid_e & 63;
-    const int hl = lane_e & 31;
-    const float L = halves_sum(l_acc);         // head hl, all keys of the split
+    const float L = halves_sum(l_acc);         // head lane & 31, all keys of the split
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
     if (!token_live) return;
     if (!live_w) {                           // (a.dst == nullptr here)
         write_empty_pairs(a, blockIdx.y, t, sp, DV, lane_e);
         return;
     }
-    const int hi4 = 4 * (lane_e >> 5);
+    const int hi4 = 4 * (lane_e >> 5), hle = lane_e & 31;
     if (a.dst != nullptr) {                  // single split: o / l in f32 straight to dst
-        const int h = hg0 + hl;
+        const int h = hg0 + hle;
         if (h < a.n_head) {
             float * d = a.dst + ((size_t)h * a.nt + t) * DV + hi4;
 #pragma unroll
@@ -270,9 +293,8 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_prefill_f16_kernel(DecodeArgs a)
     char * rec = part_record(a.part, blockIdx.y, a.nt, t, a.n_split, DV, 2);
     char * blk = rec + part_o_off(a.n_split, sp, DV, 2);
     if (lane_e < HG) {
-        const float mr = m_run[(lane_e >> 4) & 1];        // lane_e's head 16 ((lane_e >> 4) & 1) + j16
         *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, lane_e, sp)) =
-            f32x2{(mr == -INFINITY) ? -INFINITY : mr * LN2, L};                   // m in natural-log units
+            f32x2{(m_run == M_NONE) ? -INFINITY : m_run * LN2, L};                   // m in natural-log units
     }
     // o / l in f16 through this wave's staging rows [32 heads][D_v], then 16-byte row chunks out
     char * stg = ring + w * HG * C::OPITCH;
@@ -282,7 +304,7 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_prefill_f16_kernel(DecodeArgs a)
         for (int q4 = 0; q4 < 4; ++q4) {
             const half4 hv = {to_half(o[i][4 * q4] * inv), to_half(o[i][4 * q4 + 1] * inv), to_half(o[i][4 * q4 + 2] * inv),
                               to_half(o[i][4 * q4 + 3] * inv)};
-            *reinterpret_cast<half4 *>(stg + hl * C::OPITCH + (32 * i + 8 * q4 + hi4) * 2) = hv;
+            *reinterpret_cast<half4 *>(stg + hle * C::OPITCH + (32 * i + 8 * q4 + hi4) * 2) = hv;
         }
 #pragma unroll
     for (int it = 0; it < C::CPR / 2; ++it) {
