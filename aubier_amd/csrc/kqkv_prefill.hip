@@ -272,7 +272,7 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_prefill_f16_kernel(DecodeArgs a)
     const float L = halves_sum(l_acc);         // head lane & 31, all keys of the split
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
     if (!token_live) return;
-    if (!live_w) {                           // (a.dst == nullptr here)
+    if (!live_w && a.dst == nullptr) {       // (with one split a token without a live key writes zeros below)
         write_empty_pairs(a, blockIdx.y, t, sp, DV, lane_e);
         return;
     }

@@ -52,7 +52,7 @@ def runs(kind, nt, n_kv, g):
 
 
 @pytest.mark.parametrize("dk,dv", [(576, 512), (320, 256)])
-@pytest.mark.parametrize("n_kv", [65, 1088, 2500])
+@pytest.mark.parametrize("n_kv", [40, 65, 1088, 2500])
 @pytest.mark.parametrize("kind", ["causal", "edges", "some_dead", "random"])
 @pytest.mark.parametrize("split", [None, 1, 3])
 def test_live_runs(dev, dk, dv, n_kv, kind, split):
