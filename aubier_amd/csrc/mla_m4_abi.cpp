@@ -145,6 +145,33 @@ size_t q8_copy_bytes(const KqkvShape & s) {
 
 int64_t n_tiles_of(int64_t n_kv) { return (n_kv + TILE_KEYS - 1) / TILE_KEYS; }
 
+// Split count of the prefill kernel: groups x sp workgroups run one per CU, so the time goes in rounds
+// of 256 workgroups and a second round that is mostly empty costs a whole one (500 tokens x 32 heads
+// over 1,024 keys: 3 splits = 375 workgroups 83 us, 2 splits 57).  The least estimate of rounds x
+// (workgroup + tiles) + merge over 1 .. cap, in us measured on the MI355X for the two geometries: a
+// workgroup's fixed part (q in, o out), a tile, and the merge's launch and bytes (with one split the
+// kernel writes dst itself).  Measured (us, old rule ceil(256 / groups) -> this one, causal): 250
+// tokens over 1,024 keys 68 -> 47, 500 83 -> 60, 1,000 105 -> 74; over 2,048 88 -> 61, 121 -> 89,
+// 163 -> 133.
+int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t cap) {
+    const bool wide = s.dk == 576;
+    const double wg_us = wide ? 15.0 : 10.0, tile_us = wide ? 3.3 : 2.2;
+    const double out = (double)s.nt * (double)s.n_head * (double)s.dv;      // output values
+    double best = 0.0;
+    int best_sp = 1;
+    for (int64_t sp = 1; sp <= cap; ++sp) {
+        const double rounds = (double)((groups * sp + TARGET_WG - 1) / TARGET_WG);
+        double us = rounds * (wg_us + tile_us * (double)((tiles + sp - 1) / sp));
+        // records of 2 sp bytes per value read, and 4 written, at ~4 TB/s
+        us += sp > 1 ? 5.0 + out * (double)(2 * sp + 4) / 4.0e6 : out * 4.0 / 8.0e6;
+        if (sp == 1 || us < best) {
+            best = us;
+            best_sp = (int)sp;
+        }
+    }
+    return best_sp;
+}
+
 int default_splits(const KqkvShape & s) {
     // the unit a split is made of: 64-key tiles (MFMA kernels), 16-key granules (VALU kernel)
     const int64_t tiles = (use_mfma(s) || use_q8(s)) ? n_tiles_of(s.n_kv) : (s.n_kv + mla::GRAN_KEYS - 1) / mla::GRAN_KEYS;
@@ -166,6 +193,7 @@ int default_splits(const KqkvShape & s) {
     if (sp > tiles) sp = tiles;
     if (sp > MLA_M4_MAX_SPLITS) sp = MLA_M4_MAX_SPLITS;
     if (sp < 1) sp = 1;
+    if (use_prefill(s) || use_q8_prefill(s)) return prefill_splits(s, tiles, groups, sp);
     return (int)sp;
 }
 
