@@ -1,5 +1,5 @@
-// kqkv_generic.hip -- the VALU attention kernel (f32 caches and geometries outside the MFMA
-// instantiations) and the split-K merge.
+// kqkv_generic.hip -- the VALU attention kernel (geometries outside the MFMA instantiations, and f32
+// caches in few splits) and the split-K merge.
 //
 // Generic kernel: one workgroup (4 waves) per (split, head, token).  Splits are balanced runs of
 // 16-key granules (GRAN_KEYS; finer than the MFMA kernels' 64-key tiles, so that a short window

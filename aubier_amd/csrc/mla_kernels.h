@@ -78,6 +78,14 @@ hipError_t launch_q8_rows_to_f16(int dk, const char * src, int n_kv, void * dst,
 constexpr int GRAN_KEYS = 16;
 hipError_t launch_kqkv_generic(int dk, int dv, int kc_is_f16, const DecodeArgs & a, hipStream_t stream);
 
+// An f32 cache at the two MLA geometries (rows of at most F32_MAX_NB1 bytes apart: 32 rows stay within
+// a buffer's 32-bit offsets): the f32-MFMA kernel of kqkv_decode_f32.hip, 16 heads per workgroup, the
+// VALU kernel's splits and f32 records.
+constexpr int F32_HEADS = 16;
+constexpr int F32_TILE_KEYS = 32;
+constexpr int64_t F32_MAX_NB1 = 1 << 26;
+hipError_t launch_kqkv_decode_f32(int dk, int dv, const DecodeArgs & a, hipStream_t stream);
+
 // Short decode windows in one launch (kqkv_flat.hip): one workgroup per (split of <= FLAT_KEYS keys,
 // head) of one token; each writes a record (m, l, unnormalised o: dv + 4 floats) to rec
 // [head][split], and the last workgroup of each head (an agent-scope ticket per head, ticket[h],

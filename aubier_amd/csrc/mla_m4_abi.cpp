@@ -143,6 +143,26 @@ size_t q8_copy_bytes(const KqkvShape & s) {
     return use_q8_prefill(s) ? (((size_t)s.n_kv * (size_t)s.dk * 2u + 255u) & ~(size_t)255u) : 0;
 }
 
+// An f32 cache at an MLA geometry in n_split splits: the f32-MFMA kernel (16 heads per workgroup) where
+// the VALU kernel, a workgroup per (split, head, token), would run at its throughput limit of some
+// 550 workgroups or more; with fewer the VALU kernel's 16 times as many workgroups finish sooner.
+// Measured (us, VALU -> MFMA): 512 VALU workgroups (splits x heads x tokens: 16 x 32 x 1, 32 x 16 x 1,
+// 8 x 64 x 1, 4 x 32 x 4, 1 x 32 x 16) 27 -> 32, 15.4 -> 18.3, 51 -> 58, 52 -> 60, 206 -> 231 at
+// 2,048-4,096 keys; 1,024 of them 27 -> 18.6 (32 x 32), 49 -> 32 (16 x 64), 49 -> 31 (8 x 32 x 4).
+bool use_f32_mfma(const KqkvShape & s, int64_t n_split) {
+    return s.kc_type == MLA_M4_TYPE_F32 && mla::decode_f16_supported((int)s.dk, (int)s.dv) && s.kc_nb1 <= mla::F32_MAX_NB1 &&
+           n_split * s.n_head * s.nt >= 544;
+}
+// its split count: one workgroup per CU, at most one split per 32-key tile (the partial and merge of
+// 1,024 / 2,048 / 4,096 / 8,192 keys: 12.2 / 13.7 / 15.9 / 19.0 us at 32 / 64 / 128 / 128 splits, the
+// least of 16 .. 128 each)
+int64_t f32_mfma_splits(const KqkvShape & s) {
+    const int64_t groups = ((s.n_head + mla::F32_HEADS - 1) / mla::F32_HEADS) * s.nt;
+    const int64_t tiles = (s.n_kv + mla::F32_TILE_KEYS - 1) / mla::F32_TILE_KEYS;
+    const int64_t sp = (TARGET_WG + groups - 1) / groups;
+    return sp < tiles ? sp : tiles;
+}
+
 int64_t n_tiles_of(int64_t n_kv) { return (n_kv + TILE_KEYS - 1) / TILE_KEYS; }
 
 // Split count of the prefill kernel: groups x sp workgroups run one per CU, so the time goes in rounds
@@ -173,6 +193,7 @@ int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t c
 }
 
 int default_splits(const KqkvShape & s) {
+    if (use_f32_mfma(s, f32_mfma_splits(s))) return (int)f32_mfma_splits(s);
     // the unit a split is made of: 64-key tiles (MFMA kernels), 16-key granules (VALU kernel)
     const int64_t tiles = (use_mfma(s) || use_q8(s)) ? n_tiles_of(s.n_kv) : (s.n_kv + mla::GRAN_KEYS - 1) / mla::GRAN_KEYS;
     int64_t groups;   // workgroups per split
@@ -234,6 +255,7 @@ int launch_attn(const KqkvShape & s, const mla::DecodeArgs & a, hipStream_t stre
     if (f16_copy || use_prefill(s)) e = mla::launch_kqkv_prefill_f16((int)s.dk, (int)s.dv, a, stream);
     else if (use_q8(s)) e = mla::launch_kqkv_decode_q8((int)s.dk, (int)s.dv, a, stream);
     else if (use_mfma(s)) e = mla::launch_kqkv_decode_f16((int)s.dk, (int)s.dv, a, stream);
+    else if (use_f32_mfma(s, a.n_split)) e = mla::launch_kqkv_decode_f32((int)s.dk, (int)s.dv, a, stream);
     else e = mla::launch_kqkv_generic((int)s.dk, (int)s.dv, s.kc_type == MLA_M4_TYPE_F16, a, stream);
     return e == hipSuccess ? MLA_M4_OK : MLA_M4_ERR_LAUNCH;
 }

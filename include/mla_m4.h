@@ -162,7 +162,7 @@ size_t mla_m4_kqkv_workspace_bytes(const mla_m4_tensor * kcache, const mla_m4_te
  * split-K partials live in a static device array of MLA_M4_NOALLOC_SCRATCH_BYTES (32 MiB) that
  * each GPU the library runs on holds until the process ends.  With an f16 cache a 32-head group
  * at 256 splits (>= 16K keys) needs 8.45 MB per token, so decode of up to 3 tokens at H <= 32
- * fits; the f32-cache kernel uses ~256 / (H nt) splits (0.53 MB at H = 32, one token).  The
+ * fits; the f32-cache kernel uses at most 256 / (ceil(H / 16) nt) splits (8.4 MB at H = 32).  The
  * workspace a shape needs (mla_m4_kqkv_workspace_bytes, including a Q8_0 cache's f16 copy for
  * prefill) must fit the array; larger shapes (long prefill, more heads) return MLA_M4_ERR_SCRATCH.
  * Allocates nothing and calls no allocating routine; the first call on each device resolves the
@@ -184,7 +184,7 @@ int mla_m4_kqkv_default_splits(int64_t n_kv, int64_t n_head, int32_t kcache_type
  * explicit split count (1 .. MLA_M4_MAX_SPLITS).  Keys are partitioned into n_split contiguous
  * ranges of whole units, balanced (the first n_units % n_split ranges get one more unit): 64-key
  * tiles on the MFMA path (F16 cache, the two instantiated geometries; a Q8_0 cache), 16-key
- * granules on the VALU path (F32 cache, other geometries).  With a Q8_0 cache this entry point
+ * granules on the f32 and VALU paths (F32 cache, other geometries).  With a Q8_0 cache this entry point
  * always runs the 8-bit decode kernel, one pass over the window per token, also for 16 and more
  * tokens, where mla_m4_kqkv instead writes the cache's f16 values into its workspace and runs the
  * chunked-prefill kernel on them: the two agree within the f16-cache bar, not bit for bit.
