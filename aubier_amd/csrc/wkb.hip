@@ -6,7 +6,8 @@
 // Decode is a pure HBM stream of W_kb (8 MiB at d_n = 128, D_v = 512, H = 32): each wavefront
 // owns 8 (d_n = 128) or 16 (d_n = 64) consecutive rows of one head, issues all its 16-byte row
 // loads before the first use, and reduces each row over its d_n/4 lanes with xor shuffles.  For
-// a few tokens the rows stay in registers while the tokens stream past; from 16 tokens on the op
+// a few tokens the rows stay in registers while the tokens stream past, for some more the row sums run
+// on the f32 MFMA, all tokens at once (wkb_few_kernel); from 16 tokens on the op
 // is a batched GEMM and runs on MFMA (wkb_gemm_kernel, f32 operands split into f16 pieces).
 #include "mla_common.h"
 #include "mla_kernels.h"
@@ -70,6 +71,46 @@ __global__ __launch_bounds__(256) void wkb_f32_kernel(WkbArgs a) {
             }
         }
     }
+}
+
+struct __attribute__((packed, aligned(4))) F4u { float v[4]; };     // 16 bytes at dword alignment
+
+// A few tokens: 16 rows of one head per wavefront on v_mfma_f32_16x16x4_f32, whose 16 columns hold the
+// tokens, so all of them cost one pass (the kernel above reduces every row over its lanes once per
+// token).  A operand: lane (j16, g) holds W row j16's d = 16 s + 4 g + e, B: token j16's q at the same d (the k
+// order of an MFMA is free as long as both agree, so both come as 16-byte loads).  Result: rows 4 g .. +3 of token j16.
+template <int DN>
+__global__ __launch_bounds__(256) void wkb_few_kernel(WkbArgs a) {
+    constexpr int NS = DN / 16;
+    const int lane = threadIdx.x & 63;
+    const int j16 = lane & 15, g = lane >> 4;
+    const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+    if (row0 >= a.n_head * a.d_v) return;
+    const int h = row0 / a.d_v;          // d_v % 16 == 0 (host-checked): one head per wavefront
+    f32x4 wv[NS], qv[NS];
+    const float * wrow = a.w + (size_t)(row0 + j16) * DN + 4 * g;
+    const char * qrow = reinterpret_cast<const char *>(a.q) + (size_t)min(j16, a.nt - 1) * a.q_nb2 + (size_t)h * a.q_nb1 + 16 * g;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) wv[s] = *reinterpret_cast<const f32x4 *>(wrow + 16 * s);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qv[s] = *reinterpret_cast<const f32x4 *>(qrow + 64 * s);
+    __builtin_amdgcn_sched_barrier(0);   // every load in flight before the first product
+    // every product of four on an accumulator of its own, summed as a tree: as near to float64 as the row
+    // sums above (7.3e-8 relative at DN = 128; eight chains left 8.8e-8)
+    f32x4 c[4 * NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            c[4 * s + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[s][e], qv[s][e], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+    for (int n = 2 * NS; n >= 1; n /= 2)
+#pragma unroll
+        for (int i = 0; i < n; ++i) c[i] += c[i + n];
+    const f32x4 r = c[0];
+    if (j16 >= a.nt) return;
+    char * drow = reinterpret_cast<char *>(a.dst) + (size_t)j16 * a.d_nb2 + (size_t)h * a.d_nb1;
+    *reinterpret_cast<F4u *>(drow + 4 * (size_t)(row0 - h * a.d_v + 4 * g)) = F4u{{r[0], r[1], r[2], r[3]}};
 }
 
 // Many tokens (chunked prefill): per head a GEMM dst_h[t][c] = sum_d q_h[t][d] W_h[c][d] with f32
@@ -326,6 +367,16 @@ hipError_t launch_wkb_f32(const WkbArgs & a, hipStream_t stream) {
         const int64_t tiles = (int64_t)a.n_head * ((a.nt + WG_T - 1) / WG_T) * ((a.d_v + WG_T - 1) / WG_T);
         if (tiles > INT32_MAX) return hipErrorInvalidValue;
         hipLaunchKernelGGL(wkb_gemm_kernel, dim3((unsigned)tiles), dim3(256), 0, stream, a);
+        return hipGetLastError();
+    }
+    // Measured (us, a row sum per token -> all tokens at once, 32 heads, COLD): (128, 512) 5 tokens 4.65 ->
+    // 4.65, 8 5.5 -> 4.8, 15 7.8 -> 5.1 (its 64-byte row pieces stream slower than the whole rows of the
+    // other); (64, 256) 2 2.5 -> 2.9, 4 3.2 -> 2.7, 8 4.3 -> 2.7, 15 6.2 -> 2.9
+    if (a.nt >= (a.d_n == 64 ? 4 : 6) && a.nt <= 16) {
+        const dim3 grid((a.n_head * a.d_v / 16 + 3) / 4);
+        if (a.d_n == 128) hipLaunchKernelGGL(wkb_few_kernel<128>, grid, dim3(256), 0, stream, a);
+        else if (a.d_n == 64) hipLaunchKernelGGL(wkb_few_kernel<64>, grid, dim3(256), 0, stream, a);
+        else return hipErrorInvalidValue;
         return hipGetLastError();
     }
     const int total = a.n_head * a.d_v;
