@@ -27,6 +27,7 @@ namespace {
 constexpr int GTK = 64;
 constexpr int GMAX_DK = 1024;
 constexpr int GMAX_DV = 1024;
+constexpr int MLA_MAX_SPLITS_PAD = 1024;     // the largest split count (MLA_M4_MAX_SPLITS), in whole batches
 
 template <bool F16>
 __global__ __launch_bounds__(256) void kqkv_generic_kernel(DecodeArgs a, int dk, int dv) {
@@ -223,6 +224,97 @@ __global__ __launch_bounds__(256) void merge_kernel(const char * __restrict__ pa
     merge_unit<OT>(part, dv, n_split, nt, blockIdx.x, blockIdx.y, blockIdx.z, dst, sc);
 }
 
+// The PHASE merge of several tokens' f16 records (batch-of-N decode, drafted tokens): a workgroup per (256
+// columns, head, token).  With many (head, token) pairs merge_unit's folds (an exponential and a rescale
+// of 8 columns per lane and step) are the time, and each of its 64-column workgroups repeats the weights.
+// Here the weights l_s e^(m_s - m*) are taken once, a split per thread, into LDS, and the columns are
+// plain multiply-adds: 32 column lanes (8 columns each) x 8 split lanes, split lane i taking splits
+// i, i + 8, ... in batches whose loads are in flight together; a batch without a live split (the
+// regions of other sequences) is passed over.
+constexpr int MR_COLS = 256;
+__global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict__ part, int dv, int n_split, int nt,
+                                                         float * __restrict__ dst) {
+    constexpr int B = 8;                 // splits per lane and batch
+    __shared__ float wt[MLA_MAX_SPLITS_PAD];
+    __shared__ float red[2][4];
+    __shared__ __attribute__((aligned(16))) f32x4 fold[8][32][2];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int h = blockIdx.y, t = blockIdx.z, hh = h % PART_HEADS;
+    const char * rec = part_record(part, h / PART_HEADS, nt, t, n_split, dv, 2);
+    const f32x2 * ml = reinterpret_cast<const f32x2 *>(rec + part_ml_off(n_split, hh, 0));
+    const int n_pad = (n_split + 8 * B - 1) / (8 * B) * (8 * B);
+    // ---- the weights: splits tid, tid + 256, ... ----
+    constexpr int NS = MLA_MAX_SPLITS_PAD / 256;
+    f32x2 v[NS];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        const int s = tid + 256 * i;
+        v[i] = f32x2{-INFINITY, 0.0f};
+        if (256 * i < n_split) {
+            const f32x2 x = ml[min(s, n_split - 1)];
+            if (s < n_split) v[i] = x;
+        }
+        mx = fmaxf(mx, v[i][0]);
+    }
+    mx = wave_max(mx);
+    if (lane == 0) red[0][w] = mx;
+    __syncthreads();
+    const float M = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        const int s = tid + 256 * i;
+        const float f = v[i][1] * exp2_unless(v[i][0] == -INFINITY, (v[i][0] - M) * LOG2E);
+        sum += f;
+        // an empty split's block is never read: its weight says so (a live split's may underflow to 0)
+        if (s < n_pad) wt[s] = v[i][0] == -INFINITY ? -1.0f : f;
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) red[1][w] = sum;
+    __syncthreads();
+    const float L = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    // ---- the columns ----
+    const int c8 = tid & 31, sl = tid >> 5;
+    const int c = blockIdx.x * MR_COLS + 8 * c8;
+    const char * obase = rec + part_o_off(n_split, 0, dv, 2);
+    const uint32_t oblk = (uint32_t)(PART_HEADS * dv * 2);
+    const uint32_t orecs = (uint32_t)n_split * oblk;
+    const uint32_t ocol = (uint32_t)((hh * dv + c) * 2);
+    float O[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < n_pad; s0 += 8 * B) {
+        float f[B];
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            f[j] = wt[s0 + 8 * j + sl];
+            any |= f[j] >= 0.0f;
+        }
+        if (__builtin_amdgcn_ballot_w64(any) == 0) continue;
+        u32x4 x[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+            x[j] = buf_ld16<true>(obase, orecs, f[j] >= 0.0f ? (uint32_t)(s0 + 8 * j + sl) * oblk + ocol : 0xFFFFFFE0u);
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const half8 o8 = __builtin_bit_cast(half8, x[j]);
+            const float g = fmaxf(f[j], 0.0f);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) O[k] = fmaf(g, (float)o8[k], O[k]);
+        }
+    }
+    fold[sl][c8][0] = f32x4{O[0], O[1], O[2], O[3]};
+    fold[sl][c8][1] = f32x4{O[4], O[5], O[6], O[7]};
+    __syncthreads();
+    if (tid < 64) {
+        f32x4 r = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r += fold[i][tid >> 1][tid & 1];
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        *reinterpret_cast<f32x4 *>(dst + ((size_t)h * nt + t) * dv + blockIdx.x * MR_COLS + 4 * tid) = r * inv;
+    }
+}
+
 }  // namespace
 
 hipError_t launch_kqkv_generic(int dk, int dv, int kc_is_f16, const DecodeArgs & a, hipStream_t stream) {
@@ -299,6 +391,17 @@ hipError_t launch_merge(const char * part, int dv, int o_bytes, int n_split, int
             hipLaunchKernelGGL(merge_few_kernel<float>, grid, dim3(256), 0, stream, part, dv, n_split, nt, n_head, dst);
         else
             return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
+    // Several tokens (us, merge_kernel -> merge_rows_kernel, D_v 512, 32 heads, every split live): 2 tokens x
+    // 128 splits 3.7 -> 3.3, 4 x 64 4.8 -> 2.9, 8 x 128 9.1 -> 5.8, 15 x 128 14.3 -> 9.8, 8 x 256 13.3 ->
+    // 11.1; 8 x 256 with 32 live 7.6 -> 3.7.  With fewer workgroups each has more to read than merge_kernel's
+    // (2 x 256: 4.5 -> 5.4; after the partial kernel, its records cold, 2 rows x 79 splits 13.1 -> 13.6
+    // together), which stays there.
+    const int64_t wgs = (int64_t)nt * n_head * (dv / MR_COLS);
+    if (o_bytes == 2 && nt > 1 && dv % MR_COLS == 0 && n_split <= MLA_MAX_SPLITS_PAD &&
+        (wgs >= 256 || (wgs >= 192 && n_split <= 128))) {
+        hipLaunchKernelGGL(merge_rows_kernel, dim3(dv / MR_COLS, n_head, nt), dim3(256), 0, stream, part, dv, n_split, nt, dst);
         return hipGetLastError();
     }
     dim3 grid((dv + 63) / 64, n_head, nt);
