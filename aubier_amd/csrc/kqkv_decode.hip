@@ -31,7 +31,7 @@
 // Grid = (n_split, ceil(H/32), nt), 256 threads.  Output: one partial block per (32-head group,
 // token, split) -- m and l per head in f32 and the split's normalised output o/l in f16,
 // [32 heads][D_v] (mla_kernels.h) -- or, with a single split, o/l in f32 to dst.
-#include "decode_common.h"
+#include "prefill_pass.h"
 
 namespace mla {
 
@@ -160,8 +160,13 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
 // ROWS = false: row blockIdx.z (one token, the plain decode step).  ROWS = true: rows blockIdx.z,
 // blockIdx.z + gridDim.z, ... of split blockIdx.x (batch-of-N decode puts every row of the split in
 // one workgroup); with a mask, the rows that hold no live key of the split (per-sequence regions)
-// are found first, in one round trip, and only record an empty split; the others run the whole
-// pass in turn.
+// are found first, in one round trip, and only record an empty split.  The live rows go four at a time
+// through the prefill kernel's pass, which reads each K / V byte once for all four, while there are at
+// least SHARED_MIN_ROWS of them (drafted tokens over one window); one or two (regions) run the
+// whole one-row pass in turn.  Four rows over 65,536 keys in 256
+// splits of four tiles, with the merge: 69 us in turn, 48 shared; over one-tile splits the two are even
+// (35.5 and 35.3 us), and for three rows of one tile the pass is the slower one (27.9, 32.2).
+constexpr int SHARED_MIN_ROWS = 3;
 template <int DK, int DV, bool ROWS>
 __global__ __launch_bounds__(NTHR, 1) void kqkv_decode_f16_kernel(DecodeArgs a) {
     __shared__ DecodeLds<DK, DV> sh;
@@ -170,22 +175,40 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_decode_f16_kernel(DecodeArgs a) 
         return;
     }
     __shared__ uint32_t live_w[NWAVE];
+    __shared__ int live_of[NWAVE][2];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint32_t live = ~0u;
+    const int n_rows = (a.nt - (int)blockIdx.z + (int)gridDim.z - 1) / (int)gridDim.z;     // 1 .. ROWS_MAX
+    uint32_t live = (1u << n_rows) - 1u;
     if (a.nt > 1 && a.dst == nullptr && a.mask != nullptr) {
         const uint32_t bits = live_rows_of_wave<LIVE_ROUND_TILES>(a, blockIdx.x, w, lane);
         if (lane == 0) live_w[w] = bits;
         __syncthreads();
-        live = live_w[0] | live_w[1] | live_w[2] | live_w[3];
+        const uint32_t found = live_w[0] | live_w[1] | live_w[2] | live_w[3];
+        for (uint32_t dead = live & ~found; dead != 0; dead &= dead - 1)
+            if (w == 0) write_empty_pairs(a, blockIdx.y, blockIdx.z + __builtin_ctz(dead) * gridDim.z, blockIdx.x, DV, lane);
+        live &= found;
     }
-    int i = 0;
-    for (int t = blockIdx.z; t < a.nt; t += gridDim.z, ++i) {
-        if (!((live >> i) & 1u)) {
-            if (w == 0) write_empty_pairs(a, blockIdx.y, t, blockIdx.x, DV, lane);
-            continue;
+    live = __builtin_amdgcn_readfirstlane(live);
+    while (__builtin_popcount(live) >= SHARED_MIN_ROWS) {
+        // wave w takes the w-th live row (the last one again, unused, where there are only three)
+        int mine = 0;
+        bool have = false;
+#pragma unroll
+        for (int i = 0; i < NWAVE; ++i) {
+            const bool any = live != 0;
+            const int r = any ? __builtin_ctz(live) : 0;
+            if (i == w) {
+                mine = r;
+                have = any;
+            }
+            live &= live - (any ? 1u : 0u);
         }
-        decode_row<DK, DV>(a, t, sh);
+        prefill_pass<DK, DV>(a, (int)blockIdx.z + mine * (int)gridDim.z, have, sh.ring, live_of);
+        __syncthreads();                     // the next pass reuses the ring
+    }
+    for (; live != 0; live &= live - 1) {
+        decode_row<DK, DV>(a, blockIdx.z + __builtin_ctz(live) * gridDim.z, sh);
         __syncthreads();                     // the next row's q staging reuses the ring
     }
 }
