@@ -192,6 +192,27 @@ int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t c
     return best_sp;
 }
 
+// Split count of 2-15 rows on the decode kernels, from the one-row count `base` (one workgroup per CU).
+// Rows over one window (drafted tokens) all live in every split: their records, one per row and split,
+// and the passes over a split by the rows that share its workgroup are the time, so half or a quarter of
+// the splits with two or four groups of rows is faster.  Rows over regions of their own have one
+// live row per split and want the most splits, by less; the mask that tells them apart is on the device.
+// Measured (us, partial + merge, f16 cache, 32 heads; one window / regions) at 256, 128, 64 splits:
+// 16,384 keys, 2 rows 20.4/14.0, 15.7/14.1, 17.7/17.5; 4 rows 35.3/13.9, 24.2/14.3, 19.1/17.5; 8 rows
+// 60.1/14.9, 39.0/15.1, 30.1/18.2; 8,192 keys, 4 rows 30.1/13.1, 21.5/12.5, 15.7/13.5; 32,768 keys, 4
+// rows 40.4/16.8, 31.7/18.9, -; 8 rows 70.9/19.3, 46.1/19.6, -; 131,072 keys, 8 rows 122/40.3, 96/46.9;
+// 15 rows 224/63.7, 175/54.9.  So the lines lie where regions lose little.
+// Not where every row has a workgroup of its own anyway (base / tiles row groups), and not for two rows
+// over an 8-bit cache (16,384 keys 20.8/14.2 -> 17.2/15.3).
+int64_t rows_splits(const KqkvShape & s, int64_t tiles, int64_t base) {
+    const int64_t most = s.nt >= 12 ? INT64_MAX : s.nt >= 6 ? 2 * base : base;     // tiles up to here: fewer splits
+    if (tiles > most || (base + tiles - 1) / tiles >= s.nt || (s.nt == 2 && use_q8(s))) return base;
+    const int64_t half = (base + 1) / 2, quarter = (base + 3) / 4;
+    if (s.nt == 2) return half;
+    const int64_t two = tiles / 2;                                                 // two tiles a split
+    return two < quarter ? quarter : two > half ? half : two;
+}
+
 int default_splits(const KqkvShape & s) {
     if (use_f32_mfma(s, f32_mfma_splits(s))) return (int)f32_mfma_splits(s);
     // the unit a split is made of: 64-key tiles (MFMA kernels), 16-key granules (VALU kernel)
@@ -211,6 +232,7 @@ int default_splits(const KqkvShape & s) {
     // (With the records' o read by default-policy loads, which left them in the merge's L2s, fewer
     // and longer splits had won: 192 at 32,768 keys.)
     int64_t sp = (TARGET_WG + groups - 1) / groups;
+    if ((use_mfma(s) || use_q8(s)) && s.nt > 1 && s.nt < mla::PREFILL_MIN_TOKENS) sp = rows_splits(s, tiles, sp);
     if (sp > tiles) sp = tiles;
     if (sp > MLA_M4_MAX_SPLITS) sp = MLA_M4_MAX_SPLITS;
     if (sp < 1) sp = 1;
