@@ -354,38 +354,25 @@ __global__ __launch_bounds__(256) void wkb_q8_gemm_kernel(WkbArgs a) {
 }
 
 // ---- PHASE 0, KV-write ----
-// gemv: a workgroup per output row, a thread per 32-value block of the input (m4-phase.cu:95-125):
-// the thread quantises its block itself, acc = (wd * d16) * sum, the butterfly per 32 blocks, then
-// the 32-block partials summed in order.
+// gemv: a workgroup per two output rows (m4-phase.cu:95-125).  The input is quantised once per workgroup,
+// half a 32-value block per thread, into LDS; then a thread per (row, block): acc = (wd * d16) * sum, the
+// butterfly per 32 blocks, and the 32-block partials summed in order.  The row's loads go out before
+// the quantisation.  (A thread per block that quantised its own 32 values, a workgroup per row:
+// 128-byte strides between lanes, and twice the work per thread before the first dot.)
 template <int NBE>
-__global__ __launch_bounds__(NBE) void kvwrite_gemv_kernel(KvWriteArgs a) {
+__global__ __launch_bounds__(2 * NBE) void kvwrite_gemv_kernel(KvWriteArgs a) {
     // the reference's product (wd * d16) * sum and the butterfly's adds are separate statements;
     // without this the compiler fuses the first add with the product (one rounding instead of two)
 #pragma clang fp contract(off)
-    static_assert(NBE % 32 == 0 && NBE <= 1024, "whole 32-block groups");
-    __shared__ float sv[NBE / 32];
-    const int o = blockIdx.x, tid = threadIdx.x;
-    const float * xb = a.cur + 32 * tid;
-    float x[32];
-    float amax = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 32; ++k) {
-        x[k] = xb[k];
-        amax = fmaxf(amax, fabsf(x[k]));
-    }
-    const float d = amax / 127.0f;
-    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-    const float d16 = round_to_f16(d);
-    uint32_t xqw[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        uint32_t wv = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) wv |= ((uint32_t)(uint8_t)(int8_t)(int)roundf(x[4 * j + e] * id)) << (8 * e);
-        xqw[j] = wv;
-    }
+    static_assert(NBE % 32 == 0 && 2 * NBE <= 1024, "whole 32-block groups");
+    __shared__ __attribute__((aligned(16))) uint32_t xq[NBE * 8];
+    __shared__ float xd[NBE];
+    __shared__ float sv[2][NBE / 32];
+    const int tid = threadIdx.x;
+    const int r = tid >= NBE ? 1 : 0, blk = tid - r * NBE;
+    const int o = 2 * blockIdx.x + r;        // n_out is a multiple of 32
     // the block's 34 bytes: 2-byte aligned; read the 9 dwords around it and realign
-    const size_t boff = ((size_t)o * (NBE * 34)) + 34 * (size_t)tid;
+    const size_t boff = ((size_t)o * (NBE * 34)) + 34 * (size_t)blk;
     const uint32_t * bw = reinterpret_cast<const uint32_t *>(a.w + (boff & ~(size_t)3));
     const int sh = (int)(boff & 3);          // 0 or 2
     // (at sh = 0 the last two bytes of the 9th dword are the next block's: read only the 16 bits
@@ -394,21 +381,46 @@ __global__ __launch_bounds__(NBE) void kvwrite_gemv_kernel(KvWriteArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) D[i] = bw[i];
     D[8] = sh ? bw[8] : (uint32_t)*reinterpret_cast<const uint16_t *>(bw + 8);
+    // half block tid of the input
+    {
+        F4u x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const F4u *>(a.cur + 16 * tid + 4 * i);
+        float amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(x[i >> 2].v[i & 3]));
+        amax = fmaxf(amax, dpp_xor<1>(amax));
+        const float d = amax / 127.0f;
+        const float id = d != 0.0f ? 1.0f / d : 0.0f;
+        u32x4 q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t wv = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wv |= ((uint32_t)(uint8_t)(int8_t)(int)roundf(x[j].v[e] * id)) << (8 * e);
+            q[j] = wv;
+        }
+        *reinterpret_cast<u32x4 *>(xq + 4 * tid) = q;
+        if ((tid & 1) == 0) xd[tid >> 1] = round_to_f16(d);
+    }
+    __syncthreads();
     const float wd = f16_bits((D[0] >> (8 * sh)) & 0xffffu);
+    const u32x4 q0 = *reinterpret_cast<const u32x4 *>(xq + 8 * blk), q1 = *reinterpret_cast<const u32x4 *>(xq + 8 * blk + 4);
     int s = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const uint32_t qw = sh ? D[j + 1] : __builtin_amdgcn_alignbyte(D[j + 1], D[j], 2);
-        s = __builtin_amdgcn_sdot4((int)qw, (int)xqw[j], s, false);
+        const uint32_t qx = j < 4 ? q0[j & 3] : q1[j & 3];
+        s = __builtin_amdgcn_sdot4((int)qw, (int)qx, s, false);
     }
-    float acc = (wd * d16) * (float)s;
+    float acc = (wd * xd[blk]) * (float)s;
     acc = half_wave_sum(acc);
-    if ((tid & 31) == 0) sv[tid >> 5] = acc;
+    if ((blk & 31) == 0) sv[r][blk >> 5] = acc;
     __syncthreads();
-    if (tid == 0) {
-        float total = sv[0];
+    if (blk == 0) {
+        float total = sv[r][0];
 #pragma unroll
-        for (int g = 1; g < NBE / 32; ++g) total += sv[g];
+        for (int g = 1; g < NBE / 32; ++g) total += sv[r][g];
         a.dst[o] = total;
     }
 }
@@ -518,8 +530,8 @@ hipError_t launch_wvb_q8(const WvbArgs & a, hipStream_t stream) {
 hipError_t launch_kvwrite(const KvWriteArgs & a, hipStream_t stream) {
     const int n_out = a.d_lat + a.n_rope;
     if (n_out > 1024) return hipErrorInvalidValue;
-    if (a.n_embd == 4096) hipLaunchKernelGGL(kvwrite_gemv_kernel<128>, dim3(n_out), dim3(128), 0, stream, a);
-    else if (a.n_embd == 7168) hipLaunchKernelGGL(kvwrite_gemv_kernel<224>, dim3(n_out), dim3(224), 0, stream, a);
+    if (a.n_embd == 4096) hipLaunchKernelGGL(kvwrite_gemv_kernel<128>, dim3(n_out / 2), dim3(256), 0, stream, a);
+    else if (a.n_embd == 7168) hipLaunchKernelGGL(kvwrite_gemv_kernel<224>, dim3(n_out / 2), dim3(448), 0, stream, a);
     else return hipErrorInvalidValue;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
