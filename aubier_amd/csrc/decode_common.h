@@ -23,6 +23,10 @@ constexpr int WK = TK / NWAVE;  // keys per wave slice
 constexpr int HG = 32;          // heads per workgroup
 constexpr float LAZY = 15.0f;   // log2 slack before a reference max moves: P = 2^(s - m) <= 2^15,
                                 // exact in f16 (max 65504); a move rescales every accumulator
+// A moving reference is set this far (log2) below the max it moves for, so P is at most 2^8 there and a key
+// keeps f16's full precision down to 2^-22 of the largest weight: with the max itself as the reference
+// keys below 2^-14 of it fell among f16's subnormals, more of them the longer the split.
+constexpr float REF_DROP = 8.0f;
 // The lazily moved reference max of a head with no live key yet: below every finite score, so a
 // live key always moves it and exp2(s - M_NONE) of a masked key (s = -inf) is 0 without a special
 // case; a head still at M_NONE after the split had no live key (recorded as -inf).

@@ -124,8 +124,8 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
                 const bool mv = ref_moves(m_ref[n], tm[n]);
-                al[n] = !mv ? 1.0f : exp2_fast(m_ref[n] - tm[n]);      // 0 from M_NONE
-                m_ref[n] = mv ? tm[n] : m_ref[n];
+                al[n] = !mv ? 1.0f : exp2_fast(m_ref[n] - (tm[n] - REF_DROP));      // 0 from M_NONE
+                m_ref[n] = mv ? tm[n] - REF_DROP : m_ref[n];
             }
             l_acc *= al[(lane >> 4) & 1];         // this lane's head is 16 ((lane >> 4) & 1) + j16
             if (k > 0) {                          // (on the first tile the accumulators are still 0)

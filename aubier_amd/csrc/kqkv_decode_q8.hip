@@ -267,8 +267,8 @@ __device__ __forceinline__ void decode_row_q8(const DecodeArgs & a, int t, Q8Lds
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
                 const bool mv = ref_moves(m_ref[n], tm[n]);
-                al[n] = !mv ? 1.0f : exp2_fast(m_ref[n] - tm[n]);      // 0 from M_NONE
-                m_ref[n] = mv ? tm[n] : m_ref[n];
+                al[n] = !mv ? 1.0f : exp2_fast(m_ref[n] - (tm[n] - REF_DROP));      // 0 from M_NONE
+                m_ref[n] = mv ? tm[n] - REF_DROP : m_ref[n];
             }
             l_acc *= al[(lane >> 4) & 1];
             if (k > 0) {

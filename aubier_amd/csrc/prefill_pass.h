@@ -186,8 +186,8 @@ __device__ __forceinline__ void prefill_pass(const DecodeArgs & a, int t_w, bool
                 const bool mv = ref_moves(m_run, mx);
                 // a head with no live key so far holds zeros: nothing to rescale
                 const bool scale = mv && m_run != M_NONE;
-                const float al = scale ? exp2_fast(m_run - mx) : 1.0f;
-                m_run = mv ? mx : m_run;
+                const float al = scale ? exp2_fast(m_run - (mx - REF_DROP)) : 1.0f;
+                m_run = mv ? mx - REF_DROP : m_run;
                 if (__builtin_amdgcn_ballot_w64(scale) != 0) {
                     l_acc *= al;
                     // in place on the accumulator registers (kept in AGPRs); the s_nops cover the
