@@ -235,6 +235,7 @@ constexpr int MR_COLS = 256;
 __global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict__ part, int dv, int n_split, int nt,
                                                          float * __restrict__ dst) {
     constexpr int B = 8;                 // splits per lane and batch
+    constexpr float EMPTY = -1.0f;
     __shared__ float wt[MLA_MAX_SPLITS_PAD];
     __shared__ float red[2][4];
     __shared__ __attribute__((aligned(16))) f32x4 fold[8][32][2];
@@ -267,8 +268,9 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict
         const int s = tid + 256 * i;
         const float f = v[i][1] * exp2_unless(v[i][0] == -INFINITY, (v[i][0] - M) * LOG2E);
         sum += f;
-        // an empty split's block is never read: its weight says so (a live split's may underflow to 0)
-        if (s < n_pad) wt[s] = v[i][0] == -INFINITY ? -1.0f : f;
+        // an empty split's block is never read: the mark in its weight's place says so (a live split's
+        // weight is 0 or more, or NaN where its m or l is not finite, and then its block counts too)
+        if (s < n_pad) wt[s] = v[i][0] == -INFINITY ? EMPTY : f;
     }
     sum = wave_sum(sum);
     if (lane == 0) red[1][w] = sum;
@@ -288,17 +290,17 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict
 #pragma unroll
         for (int j = 0; j < B; ++j) {
             f[j] = wt[s0 + 8 * j + sl];
-            any |= f[j] >= 0.0f;
+            any |= f[j] != EMPTY;
         }
         if (__builtin_amdgcn_ballot_w64(any) == 0) continue;
         u32x4 x[B];
 #pragma unroll
         for (int j = 0; j < B; ++j)
-            x[j] = buf_ld16<true>(obase, orecs, f[j] >= 0.0f ? (uint32_t)(s0 + 8 * j + sl) * oblk + ocol : 0xFFFFFFE0u);
+            x[j] = buf_ld16<true>(obase, orecs, f[j] != EMPTY ? (uint32_t)(s0 + 8 * j + sl) * oblk + ocol : 0xFFFFFFE0u);
 #pragma unroll
         for (int j = 0; j < B; ++j) {
             const half8 o8 = __builtin_bit_cast(half8, x[j]);
-            const float g = fmaxf(f[j], 0.0f);
+            const float g = f[j] != EMPTY ? f[j] : 0.0f;
 #pragma unroll
             for (int k = 0; k < 8; ++k) O[k] = fmaf(g, (float)o8[k], O[k]);
         }
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict
         f32x4 r = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 8; ++i) r += fold[i][tid >> 1][tid & 1];
-        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        const float inv = M == -INFINITY ? 0.0f : 1.0f / L;     // 0 only if every split is empty
         *reinterpret_cast<f32x4 *>(dst + ((size_t)h * nt + t) * dv + blockIdx.x * MR_COLS + 4 * tid) = r * inv;
     }
 }
