@@ -475,6 +475,9 @@ __device__ __forceinline__ void slice_scores(const DecodeArgs & a, const f32x4 &
 // lanes' own maxima first and takes the cross-lane max only on the (rare) path where some reference
 // moves.
 __device__ __forceinline__ bool ref_moves(float m, float x) { return x > m + LAZY; }
+// min(x, LAZY) that lets a NaN through (v_minimum3_f32): fminf made the weight of a NaN score 2^15, and
+// the token came out as a finite average around that key.
+__device__ __forceinline__ float clamp_p(float x) { return __builtin_elementwise_minimum(x, LAZY); }
 
 // ---------------------------------------------------------------- the decode kernels
 // (kqkv_decode.hip, and the 8-bit cache kernel of kqkv_decode_q8.hip)
@@ -580,7 +583,7 @@ __device__ __forceinline__ void decode_epilogue(const DecodeArgs & a, char * stg
     if (w == 0 && lane_e < HG) {
         const float mr = m_ref[(lane_e >> 4) & 1];        // lane_e's head 16 ((lane_e >> 4) & 1) + j16
         *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, lane_e, sp)) =
-            f32x2{(mr == M_NONE) ? -INFINITY : mr * LN2, L};                      // m in natural-log units
+            f32x2{(mr == M_NONE) ? -INFINITY : mr * LN2, (mr == M_NONE) ? 0.0f : L};     // m in natural-log units
     }
     // o / l in f16 through stg, LDS of this wave's own that no wave reads any more (at least
     // HG * OPITCH bytes), as [32 heads][DVQ] rows; then 16-byte chunks out, 4 head rows of 2 * DVQ

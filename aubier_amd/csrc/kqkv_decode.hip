@@ -99,7 +99,7 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
                 half4 ph;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    ph[r] = to_half(exp2_fast(fminf(sc[n][r] - m_ref[n], 15.0f)));     // masked: 2^-inf = 0
+                    ph[r] = to_half(exp2_fast(clamp_p(sc[n][r] - m_ref[n])));     // masked: 2^-inf = 0
                 *reinterpret_cast<half4 *>(&pxv[(16 * n + j16) * C::PROW + WK * w + 4 * g]) = ph;
             }
         };

@@ -244,7 +244,7 @@ __device__ __forceinline__ void decode_row_q8(const DecodeArgs & a, int t, Q8Lds
             for (int n = 0; n < 2; ++n) {
                 half4 ph;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ph[r] = to_half(exp2_fast(fminf(sc[n][r] - m_ref[n], 15.0f)));
+                for (int r = 0; r < 4; ++r) ph[r] = to_half(exp2_fast(clamp_p(sc[n][r] - m_ref[n])));
                 *reinterpret_cast<half4 *>(&sh.px[(16 * n + j16) * C::PROW + WK * w + 4 * g]) = ph;
             }
         };

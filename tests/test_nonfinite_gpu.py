@@ -53,10 +53,10 @@ def test_nonfinite_stays(dev, dk, dv, cache, nt, split):
     assert torch.equal(out, clean)
 
     kc_nan = kc.clone()
-    if cache == "q8":
-        kc_nan[N_KV - 5, 34:36] = torch.tensor([0x00, 0x7e], dtype=torch.uint8)     # block 1's scale, values 32 .. 63
+    if cache == "q8":                            # the scale of the block that holds the first rope values
+        kc_nan[N_KV - 5, dv // 32 * 34:dv // 32 * 34 + 2] = torch.tensor([0x00, 0x7e], dtype=torch.uint8)
     else:
-        kc_nan[N_KV - 5, 32] = math.nan
+        kc_nan[N_KV - 5, dv] = math.nan
     out = kqkv(kc_nan, dk, q, mask, split, dv, dev)
-    assert not torch.isfinite(out[:, nt - 1, 32]).any()
+    assert not torch.isfinite(out[:, nt - 1]).any()          # V is finite: only the score is NaN
     assert torch.equal(out[:, :nt - 1], clean[:, :nt - 1])
