@@ -475,9 +475,6 @@ __device__ __forceinline__ void slice_scores(const DecodeArgs & a, const f32x4 &
 // lanes' own maxima first and takes the cross-lane max only on the (rare) path where some reference
 // moves.
 __device__ __forceinline__ bool ref_moves(float m, float x) { return x > m + LAZY; }
-// min(x, LAZY) that lets a NaN through (v_minimum3_f32): fminf made the weight of a NaN score 2^15, and
-// the token came out as a finite average around that key.
-__device__ __forceinline__ float clamp_p(float x) { return __builtin_elementwise_minimum(x, LAZY); }
 
 // ---------------------------------------------------------------- the decode kernels
 // (kqkv_decode.hip, and the 8-bit cache kernel of kqkv_decode_q8.hip)

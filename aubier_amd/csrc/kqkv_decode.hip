@@ -90,8 +90,9 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
         else qk_slice<DK, false>(ss, dn, sb, lane, qreg, s0, s1);
         float sc[2][4], mx[2];
         slice_scores(a, slice_mask<DK>(sb, lane), kbase, lane, s0, s1, sc, mx);
-        // P against the current reference (exact unless the reference moves below; the clamp only
-        // keeps a provisional value finite), into the exchange as [32 heads][64 keys]
+        // P against the current reference, into the exchange as [32 heads][64 keys].  Where the
+        // reference moves below it is written again before any read, so a provisional value may
+        // overflow; it is not clamped, as fminf would give a NaN score the weight of its bound.
         half_t * pxv = px[par];
         auto put_p = [&]() {
 #pragma unroll
@@ -99,7 +100,7 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
                 half4 ph;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    ph[r] = to_half(exp2_fast(clamp_p(sc[n][r] - m_ref[n])));     // masked: 2^-inf = 0
+                    ph[r] = to_half(exp2_fast(sc[n][r] - m_ref[n]));     // masked: 2^-inf = 0
                 *reinterpret_cast<half4 *>(&pxv[(16 * n + j16) * C::PROW + WK * w + 4 * g]) = ph;
             }
         };

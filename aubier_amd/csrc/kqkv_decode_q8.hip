@@ -237,14 +237,14 @@ __device__ __forceinline__ void decode_row_q8(const DecodeArgs & a, int t, Q8Lds
         const int kbase = (ss.t0 + k) * TK + WK * w;
         float sc[2][4], mx[2];
         slice_scores(a, mk, kbase, lane, s0, s1, sc, mx);
-        // P against the current reference (exact unless it moves below; the clamp only keeps a
-        // provisional value finite), into the exchange as [32 heads][64 keys]
+        // P against the current reference (written again where it moves below, so a provisional
+        // value may overflow; a NaN stays one), into the exchange as [32 heads][64 keys]
         auto put_p = [&]() {
 #pragma unroll
             for (int n = 0; n < 2; ++n) {
                 half4 ph;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ph[r] = to_half(exp2_fast(clamp_p(sc[n][r] - m_ref[n])));
+                for (int r = 0; r < 4; ++r) ph[r] = to_half(exp2_fast(sc[n][r] - m_ref[n]));
                 *reinterpret_cast<half4 *>(&sh.px[(16 * n + j16) * C::PROW + WK * w + 4 * g]) = ph;
             }
         };
