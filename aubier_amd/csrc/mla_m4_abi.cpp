@@ -165,25 +165,57 @@ int64_t f32_mfma_splits(const KqkvShape & s) {
 
 int64_t n_tiles_of(int64_t n_kv) { return (n_kv + TILE_KEYS - 1) / TILE_KEYS; }
 
+int64_t n_groups_of(int64_t n_head) { return (n_head + MLA_M4_PART_HEADS - 1) / MLA_M4_PART_HEADS; }
+
+int part_o_bytes(const KqkvShape & s) { return s.kc_type == MLA_M4_TYPE_F32 ? 4 : 2; }     // f16 o for F16 and Q8_0 caches
+
+int64_t part_floats(const KqkvShape & s) { return (int64_t)(mla::part_block_bytes((int)s.dv, part_o_bytes(s)) / 4); }
+
+size_t part_bytes(const KqkvShape & s, int n_split) {
+    return (size_t)n_groups_of(s.n_head) * (size_t)s.nt * (size_t)n_split * mla::part_block_bytes((int)s.dv, part_o_bytes(s));
+}
+
 // Split count of the prefill kernel: groups x sp workgroups run one per CU, so the time goes in rounds
 // of 256 workgroups and a second round that is mostly empty costs a whole one (500 tokens x 32 heads
-// over 1,024 keys: 3 splits = 375 workgroups 83 us, 2 splits 57).  The least estimate of rounds x
-// (workgroup + tiles) + merge over 1 .. cap, in us measured on the MI355X for the two geometries: a
-// workgroup's fixed part (q in, o out), a tile, and the merge's launch and bytes (with one split the
-// kernel writes dst itself).  Measured (us, old rule ceil(256 / groups) -> this one, causal): 250
-// tokens over 1,024 keys 68 -> 47, 500 83 -> 60, 1,000 105 -> 74; over 2,048 88 -> 61, 121 -> 89,
-// 163 -> 133.
+// over 1,024 keys: 3 splits = 375 workgroups 83 us, 2 splits 57).  The least estimate over 1 .. cap of
+//   rounds x (round + (tile + load x share of the CUs in use) x tiles) + the end,
+// in us, the constants fitted for each geometry to KQKV at 16-1,000 tokens x 32 heads over 16-5,096 keys
+// and every split count (224 shapes; the chosen count is on average 1% slower than the best one).  The
+// end with one split is dst written by the attention kernel itself, in 16-byte pieces of rows 2 KB apart, less
+// 1.4 us (D_k 576) and 2.5 (320) for the launch it saves a pass of several ops; with more, records of
+// 2 sp bytes per output value read and 4 written, and the merge, a loop over the splits up to 16 of them,
+// their shares across a workgroup's lanes beyond.
+// One split is right from some 600 tokens on, where two make a second round; below, two or three are faster
+// also over one or two tiles each (us, 1 split -> the chosen): 152 tokens over 252 keys 35.1 -> 29.7, 192
+// over 292 38.0 -> 32.3, 400 over 500 47.0 -> 41.3; D_k 320, 320 over 420 29.3 -> 25.2.  Against
+// ceil(256 / groups) splits: 400 over 1,000 keys 72 -> 55, 96 over 696 53 -> 31, 1,000 over 1,000 107 -> 74.
+struct PrefillCost {
+    double round, tile, load;            // per round, per tile, per tile at full load
+    double direct, direct_val;           // one split: fixed, per million output values
+    double few, few_split, many, mbyte;  // merge: fixed and per split up to 16 splits; fixed beyond; per MB
+};
+constexpr int PREFILL_FEW_SPLITS = 16;
+// Records beyond mla_m4_kqkv_noalloc's array are taken where a split has at least this many tiles (and a
+// merge of few splits): below, a smaller count is near as fast and keeps the call open to that entry
+// point (256 tokens over 856 keys 45.5 us at four splits, 44.0 at three; 512 over 612 47.7 and 52.7).
+constexpr int PREFILL_BIG_TILES = 6;
 int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t cap) {
-    const bool wide = s.dk == 576;
-    const double wg_us = wide ? 15.0 : 10.0, tile_us = wide ? 3.3 : 2.2;
-    const double out = (double)s.nt * (double)s.n_head * (double)s.dv;      // output values
+    static constexpr PrefillCost WIDE = {3.5, 3.1, 0.29, 15.6, 0.11, 12.0, 0.56, 16.0, 0.13};
+    static constexpr PrefillCost NARROW = {3.4, 2.5, 0.10, 7.0, 0.41, 9.7, 0.55, 9.6, 0.21};
+    const PrefillCost & c = s.dk == 576 ? WIDE : NARROW;
+    const double mval = 1e-6 * (double)s.nt * (double)s.n_head * (double)s.dv;      // million output values
     double best = 0.0;
     int best_sp = 1;
     for (int64_t sp = 1; sp <= cap; ++sp) {
-        const double rounds = (double)((groups * sp + TARGET_WG - 1) / TARGET_WG);
-        double us = rounds * (wg_us + tile_us * (double)((tiles + sp - 1) / sp));
-        // records of 2 sp bytes per value read, and 4 written, at ~4 TB/s
-        us += sp > 1 ? 5.0 + out * (double)(2 * sp + 4) / 4.0e6 : out * 4.0 / 8.0e6;
+        if (sp > 1 && part_bytes(s, (int)sp) > MLA_M4_NOALLOC_SCRATCH_BYTES &&
+            (sp > PREFILL_FEW_SPLITS || tiles < PREFILL_BIG_TILES * sp))
+            continue;
+        const int64_t wgs = groups * sp;
+        const double rounds = (double)((wgs + TARGET_WG - 1) / TARGET_WG);
+        const double share = wgs < TARGET_WG ? (double)wgs / TARGET_WG : 1.0;
+        double us = rounds * (c.round + (c.tile + c.load * share) * (double)((tiles + sp - 1) / sp));
+        if (sp == 1) us += c.direct + c.direct_val * mval;
+        else us += (sp <= PREFILL_FEW_SPLITS ? c.few + c.few_split * (double)sp : c.many) + c.mbyte * mval * (double)(2 * sp + 4);
         if (sp == 1 || us < best) {
             best = us;
             best_sp = (int)sp;
@@ -238,16 +270,6 @@ int default_splits(const KqkvShape & s) {
     if (sp < 1) sp = 1;
     if (use_prefill(s) || use_q8_prefill(s)) return prefill_splits(s, tiles, groups, sp);
     return (int)sp;
-}
-
-int64_t n_groups_of(int64_t n_head) { return (n_head + MLA_M4_PART_HEADS - 1) / MLA_M4_PART_HEADS; }
-
-int part_o_bytes(const KqkvShape & s) { return s.kc_type == MLA_M4_TYPE_F32 ? 4 : 2; }     // f16 o for F16 and Q8_0 caches
-
-int64_t part_floats(const KqkvShape & s) { return (int64_t)(mla::part_block_bytes((int)s.dv, part_o_bytes(s)) / 4); }
-
-size_t part_bytes(const KqkvShape & s, int n_split) {
-    return (size_t)n_groups_of(s.n_head) * (size_t)s.nt * (size_t)n_split * mla::part_block_bytes((int)s.dv, part_o_bytes(s));
 }
 
 mla::DecodeArgs make_args(const mla_m4_tensor * kc, const mla_m4_tensor * q, const mla_m4_tensor * mask,
