@@ -162,12 +162,13 @@ __device__ __forceinline__ void decode_row(const DecodeArgs & a, int t, DecodeLd
 // blockIdx.z + gridDim.z, ... of split blockIdx.x (batch-of-N decode puts every row of the split in
 // one workgroup); with a mask, the rows that hold no live key of the split (per-sequence regions)
 // are found first, in one round trip, and only record an empty split.  The live rows go four at a time
-// through the prefill kernel's pass, which reads each K / V byte once for all four, while there are at
-// least SHARED_MIN_ROWS of them (drafted tokens over one window); one or two (regions) run the
-// whole one-row pass in turn.  Four rows over 65,536 keys in 256
-// splits of four tiles, with the merge: 69 us in turn, 48 shared; over one-tile splits the two are even
-// (35.5 and 35.3 us), and for three rows of one tile the pass is the slower one (27.9, 32.2).
-constexpr int SHARED_MIN_ROWS = 3;
+// through the prefill kernel's pass, which reads each K / V byte once for all four, while at least four
+// are left, or three in a split of two tiles or more (drafted tokens over one window); fewer (regions) run
+// the whole one-row pass in turn.  WKB, partial and merge in us a layer, three live rows in turn -> shared:
+// three rows over 65,536 keys (splits of four tiles) 60.5 -> 49.2, 49,152 (three) 52.7 -> 45.5, 32,768
+// (two) 44.1 -> 41.5, six over 16,384 (two groups, two tiles) 39.5 -> 40.2; of one tile (11 rows over 4,096
+// keys, four groups) 31.9 -> 35.5.  Four rows of one tile are even (35.5 and 35.3 with the merge).  By default
+// four rows over 16,384 keys run as two groups of two rows (rows_splits), in turn.
 template <int DK, int DV, bool ROWS>
 __global__ __launch_bounds__(NTHR, 1) void kqkv_decode_f16_kernel(DecodeArgs a) {
     __shared__ DecodeLds<DK, DV> sh;
@@ -191,7 +192,9 @@ __global__ __launch_bounds__(NTHR, 1) void kqkv_decode_f16_kernel(DecodeArgs a) 
         live &= found;
     }
     live = __builtin_amdgcn_readfirstlane(live);
-    while (__builtin_popcount(live) >= SHARED_MIN_ROWS) {
+    const int n_my = a.n_tiles / a.n_split + ((int)blockIdx.x < a.n_tiles % a.n_split ? 1 : 0);   // tiles of this split
+    const int min_rows = n_my > 1 ? 3 : 4;
+    while (__builtin_popcount(live) >= min_rows) {
         // wave w takes the w-th live row (the last one again, unused, where there are only three)
         int mine = 0;
         bool have = false;
