@@ -205,8 +205,9 @@ __global__ __launch_bounds__(256) void kqkv_generic_kernel(DecodeArgs a, int dk,
     char * rec = part_record(a.part, h / PART_HEADS, a.nt, t, a.n_split, dv, OB);
     const int hh = h % PART_HEADS;
     char * blk = rec + part_o_off(a.n_split, sp, dv, OB);
-    if (tid == 0)
-        *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) = f32x2{(m_run == -INFINITY) ? -INFINITY : m_run * LN2, l_run};
+    if (tid == 0)                    // l = 0 with no live key, also where masked keys left it NaN
+        *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) =
+            (m_run == -INFINITY) ? f32x2{-INFINITY, 0.0f} : f32x2{m_run * LN2, l_run};
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     if (writer) {
         const f32x4 r = o * inv;
