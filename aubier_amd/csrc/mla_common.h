@@ -14,6 +14,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+struct __attribute__((packed, aligned(4))) F4u { float v[4]; };      // 16 bytes at dword alignment
 
 constexpr int WAVE = 64;
 constexpr float LOG2E = 1.4426950408889634f;

@@ -197,7 +197,7 @@ struct PrefillCost {
 constexpr int PREFILL_FEW_SPLITS = 16;
 // Records beyond mla_m4_kqkv_noalloc's array are taken where a split has at least this many tiles (and a
 // merge of few splits): below, a smaller count is near as fast and keeps the call open to that entry
-// point (256 tokens over 856 keys 45.5 us at four splits, 44.0 at three; 512 over 612 47.7 and 52.7).
+// point (256 tokens over 856 keys 45.5 us at four splits, 44.0 at three; 512 over 612 47.7 at two, 52.7 at one).
 constexpr int PREFILL_BIG_TILES = 6;
 int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t cap) {
     static constexpr PrefillCost WIDE = {3.5, 3.1, 0.29, 15.6, 0.11, 12.0, 0.56, 16.0, 0.13};
@@ -233,9 +233,17 @@ int prefill_splits(const KqkvShape & s, int64_t tiles, int64_t groups, int64_t c
 // 16,384 keys, 2 rows 20.4/14.0, 15.7/14.1, 17.7/17.5; 4 rows 35.3/13.9, 24.2/14.3, 19.1/17.5; 8 rows
 // 60.1/14.9, 39.0/15.1, 30.1/18.2; 8,192 keys, 4 rows 30.1/13.1, 21.5/12.5, 15.7/13.5; 32,768 keys, 4
 // rows 40.4/16.8, 31.7/18.9, -; 8 rows 70.9/19.3, 46.1/19.6, -; 131,072 keys, 8 rows 122/40.3, 96/46.9;
-// 15 rows 224/63.7, 175/54.9.  So the lines lie where regions lose little.
+// 15 rows 224/63.7, 175/54.9.  So the lines lie where regions lose little.  What both lose and gain by
+// the rule (us a layer, WKB, partial and merge; one window / regions, base -> this count): f16 cache, 2 rows
+// over 16,384 keys 27.2/18.5 -> 21.0/19.6, 3 over 8,192 25.1/17.6 -> 19.9/19.2, 4 over 16,384 41.4/19.6 ->
+// 31.0/20.7, 8 over 32,768 84.1/24.7 -> 54.3/25.9, 15 over 65,536 177/34.7 -> 125/38.5; 8-bit cache, whose
+// rows dequantise a tile each for themselves, 3 over 8,192 25.3/17.8 -> 21.3/20.3, 3 over 16,384 34.4/20.4
+// -> 30.8/20.7, 4 over 16,384 42.4/20.0 -> 32.7/21.4, 8 over 32,768 93.6/25.3 -> 69.0/27.4, 15 over
+// 65,536 228/35.5 -> 194/40.8.  Error against float64: up to 2% more with fewer splits (batch of 8 over
+// 32,768 cells 3.58e-4 -> 3.66e-4): the largest weight of a split's first tile is a power of two, exact in f16,
+// and a longer split has more keys beside it.
 // Not where every row has a workgroup of its own anyway (base / tiles row groups), and not for two rows
-// over an 8-bit cache (16,384 keys 20.8/14.2 -> 17.2/15.3).
+// over an 8-bit cache (16,384 keys 26.5/18.6 at 256 splits, 21.8/20.6 at 128).
 int64_t rows_splits(const KqkvShape & s, int64_t tiles, int64_t base) {
     const int64_t most = s.nt >= 12 ? INT64_MAX : s.nt >= 6 ? 2 * base : base;     // tiles up to here: fewer splits
     if (tiles > most || (base + tiles - 1) / tiles >= s.nt || (s.nt == 2 && use_q8(s))) return base;
@@ -450,7 +458,10 @@ void * scratch_ptr() {
 // heads, D_k 576): F32 cache 64 / 256 / 512 keys 9.85 / 11.46 / 15.10 us against 14.11 / 14.40 /
 // 15.50 us for split-K partial + merge; F16 cache 64 / 256 keys 10.37 / 11.51 us against
 // 12.73 / 13.18 us, but 512 keys 14.78 against 13.46 (every head's workgroups re-read the split's
-// rows, and the MFMA kernel reads them once), hence the F16 bound.
+// rows, and the MFMA kernel reads them once), hence the F16 bound.  The F32 bound is that of 32 heads and
+// the VALU kernel (384 keys 14.1 against 16.2 us, 512 16.3 against 16.1).  From 544 (split, head) pairs
+// split-K runs on the f32-MFMA kernel, and more heads meet it earlier: 40 heads 256 / 384 / 512 keys 13.3 /
+// 15.1 / 19.1 us against 18.5 / 19.2 / 18.0, 64 heads 15.5 / 19.5 / 24.1 against 18.1 / 19.3 / 19.3.
 constexpr int FLAT_MAX_HEADS = 256;
 constexpr int FLAT_F16_MAX_KEYS = 256;
 bool flat_eligible(const KqkvShape & s) {

@@ -139,8 +139,7 @@ inline bool wkb_q8_tiled(const WkbArgs & a) {
 constexpr int GT = 32;                   // tokens per workgroup
 constexpr uint32_t Q_PAD = 16;           // LDS row padding: rows start on distinct banks
 
-struct __attribute__((packed, aligned(4))) F4u { float v[4]; };       // 16 bytes at dword alignment
-struct __attribute__((packed, aligned(4))) U4u { uint32_t v[4]; };
+struct __attribute__((packed, aligned(4))) U4u { uint32_t v[4]; };       // as F4u
 
 // Half a Q8 block of token r = lane & 31 (values 16 (lane >> 5) .. +15 of the block at x): its int8
 // quants as 4 dwords and the block's scale, with quant_lane's arithmetic (the two halves of a block

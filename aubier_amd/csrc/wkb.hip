@@ -73,8 +73,6 @@ __global__ __launch_bounds__(256) void wkb_f32_kernel(WkbArgs a) {
     }
 }
 
-struct __attribute__((packed, aligned(4))) F4u { float v[4]; };     // 16 bytes at dword alignment
-
 // A few tokens: 16 rows of one head per wavefront on v_mfma_f32_16x16x4_f32, whose 16 columns hold the
 // tokens, so all of them cost one pass (the kernel above reduces every row over its lanes once per
 // token).  A operand: lane (j16, g) holds W row j16's d = 16 s + 4 g + e, B: token j16's q at the same d (the k
@@ -372,7 +370,7 @@ hipError_t launch_wkb_f32(const WkbArgs & a, hipStream_t stream) {
     // Measured (us, a row sum per token -> all tokens at once, 32 heads, COLD): (128, 512) 5 tokens 4.65 ->
     // 4.65, 8 5.5 -> 4.8, 15 7.8 -> 5.1 (its 64-byte row pieces stream slower than the whole rows of the
     // other); (64, 256) 2 2.5 -> 2.9, 4 3.2 -> 2.7, 8 4.3 -> 2.7, 15 6.2 -> 2.9
-    if (a.nt >= (a.d_n == 64 ? 4 : 6) && a.nt <= 16) {
+    if (a.nt >= (a.d_n == 64 ? 4 : 6) && a.nt < WKB_GEMM_MIN_TOKENS) {
         const dim3 grid((a.n_head * a.d_v / 16 + 3) / 4);
         if (a.d_n == 128) hipLaunchKernelGGL(wkb_few_kernel<128>, grid, dim3(256), 0, stream, a);
         else if (a.d_n == 64) hipLaunchKernelGGL(wkb_few_kernel<64>, grid, dim3(256), 0, stream, a);

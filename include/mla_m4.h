@@ -162,7 +162,9 @@ size_t mla_m4_kqkv_workspace_bytes(const mla_m4_tensor * kcache, const mla_m4_te
  * split-K partials live in a static device array of MLA_M4_NOALLOC_SCRATCH_BYTES (32 MiB) that
  * each GPU the library runs on holds until the process ends.  With an f16 cache a 32-head group
  * at 256 splits (>= 16K keys) needs 8.45 MB per token, so decode of up to 3 tokens at H <= 32
- * fits; the f32-cache kernel uses at most 256 / (ceil(H / 16) nt) splits (8.4 MB at H = 32).  The
+ * fits; an f32 cache takes ceil(256 / (ceil(H / 16) nt)) splits at most, which always fits: at D_v = 512
+ * 8.4 MB for one token at H = 32, 16.8 MB at H <= 16, 33.55 MB (512 bytes below the array's size) for
+ * 255 tokens at H <= 16.  The
  * workspace a shape needs (mla_m4_kqkv_workspace_bytes, including a Q8_0 cache's f16 copy for
  * prefill) must fit the array; larger shapes (long prefill, more heads) return MLA_M4_ERR_SCRATCH.
  * Allocates nothing and calls no allocating routine; the first call on each device resolves the
@@ -174,9 +176,11 @@ int mla_m4_kqkv_noalloc(const mla_m4_tensor * kcache, const mla_m4_tensor * q,
                         const mla_m4_tensor * mask, float kq_scale, const mla_m4_tensor * dst, void * stream);
 
 /* Split count mla_m4_kqkv uses for a decode window of n_kv keys (a function of the window): about
- * one workgroup per CU, at most one split per 64-key tile (one token over an f16 cache: one tile per
- * split up to 256 tiles, then 256 splits -- also the fastest choice for the whole op, partial then
- * merge, measured over 2K-64K keys). */
+ * one workgroup per CU, at most one split per 64-key tile, or per 32-key tile of an f32 cache (one token
+ * over an f16 cache: one tile per split up to 256 tiles, then 256 splits -- also the fastest choice for
+ * the whole op, partial then merge, measured over 2K-64K keys).  For one token: 2-15 tokens use down to a
+ * quarter of it, which suits tokens that share a window (16K keys, 4 tokens: 25% faster) and costs tokens
+ * with regions of their own some 5%; 16 and more have a rule of their own. */
 int mla_m4_kqkv_default_splits(int64_t n_kv, int64_t n_head, int32_t kcache_type);
 
 /* -------------------------------------------------------------------------------------------

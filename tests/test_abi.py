@@ -154,6 +154,14 @@ def test_default_splits_and_workspace(lib):
     assert A.kqkv_workspace_bytes(kc, q2, torch.zeros((32, 2, 512))) == 0      # two tokens, one tile: one split
 
 
+def test_f32_cache_records_fit_the_no_alloc_array():
+    kc = torch.empty((4096 * 4, 576))
+    for H in (1, 8, 9, 16, 17, 32, 33, 40, 48, 64, 128, 255):
+        for nt in (1, 2, 3, 5, 8, 17, 33, 51, 64, 85, 86, 127, 128, 129, 170, 255, 256, 300):
+            need = A.kqkv_workspace_bytes(kc, torch.empty((nt, H, 576)), torch.empty((H, nt, 512)))
+            assert need <= ops.NOALLOC_SCRATCH_BYTES, (H, nt, need)
+
+
 def test_entry_points_reject_before_launching(lib):
     kc, q, mask, out = decode_tensors()
     vk, vq, vm, vo = (ops.view(t) for t in (kc, q, mask, out))

@@ -1,8 +1,7 @@
 """Register / scratch / LDS budgets of every kernel, from the compiler's own resource report
 (`-Rpass-analysis=kernel-resource-usage`), the check the reference runs on each build
 (patches/ggml-m4/m4-kqkv.cu:39-42; ggml-hip/CMakeLists.txt:116-118).  A spill in a streaming
-loop costs more than the kernel's arithmetic, so the hot kernels are held at zero VGPR spills;
-the prefill kernel's few spills sit in its epilogue (outside the tile loop) and are capped.
+loop costs more than the kernel's arithmetic, so the kernels are held at zero VGPR spills.
 CPU-only: hipcc cross-compiles for gfx950 here."""
 import concurrent.futures as cf
 import re
@@ -22,16 +21,21 @@ LDS_MAX = 160 * 1024
 BUDGET = {
     "kqkv_decode_f16_kernel": (0, 0),
     "kqkv_decode_q8_kernel": (0, 0),
-    "kqkv_prefill_f16_kernel": (24, 128),
+    "kqkv_decode_f32_kernel": (0, 0),
+    "kqkv_prefill_f16_kernel": (0, 0),
     "kqkv_generic_kernel": (0, 0),
     "kqkv_flat_kernel": (0, 0),
     "q8_rows_to_f16_kernel": (0, 0),
     "merge_kernel": (0, 0),
+    "merge_rows_kernel": (0, 0),
     "merge_few_kernel": (0, 0),
     "wkb_f32_kernel": (0, 0),
+    "wkb_few_kernel": (0, 0),
     "wkb_gemm_kernel": (0, 0),
     "wkb_q8_kernel": (0, 0),
+    "wkb_q8_gemm_kernel": (0, 0),
     "wvb_q8_kernel": (0, 0),
+    "wvb_q8_gemm_kernel": (0, 0),
     "kvwrite_gemv_kernel": (0, 0),
     "kvwrite_tail_kernel": (0, 0),
 }
