@@ -579,8 +579,14 @@ __device__ __forceinline__ void decode_epilogue(const DecodeArgs & a, char * stg
     char * blk = rec + part_o_off(a.n_split, sp, DV, 2);
     if (w == 0 && lane_e < HG) {
         const float mr = m_ref[(lane_e >> 4) & 1];        // lane_e's head 16 ((lane_e >> 4) & 1) + j16
+        float lr = L;
+        if (mr == M_NONE && L != L) {                     // (see any_live_key)
+            const int base_t = a.n_tiles / a.n_split, rem = a.n_tiles % a.n_split;
+            const int t0 = sp * base_t + min(sp, rem);
+            if (!any_live_key(a, t, t0 * TK, min((t0 + base_t + (sp < rem ? 1 : 0)) * TK, a.n_kv))) lr = 0.0f;
+        }
         *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, lane_e, sp)) =
-            f32x2{(mr == M_NONE) ? -INFINITY : mr * LN2, (mr == M_NONE) ? 0.0f : L};     // m in natural-log units
+            f32x2{(mr == M_NONE) ? -INFINITY : mr * LN2, lr};                      // m in natural-log units
     }
     // o / l in f16 through stg, LDS of this wave's own that no wave reads any more (at least
     // HG * OPITCH bytes), as [32 heads][DVQ] rows; then 16-byte chunks out, 4 head rows of 2 * DVQ

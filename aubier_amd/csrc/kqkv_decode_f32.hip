@@ -197,9 +197,11 @@ __global__ __launch_bounds__(256, 1) void kqkv_decode_f32_kernel(DecodeArgs a) {
     } else {
         const int hh = h % PART_HEADS;
         char * rec = part_record(a.part, h / PART_HEADS, a.nt, t, a.n_split, DV, 4);
-        if (w == 0 && g == 0)            // l = 0 with no live key, also where masked keys left it NaN
-            *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) =
-                (m_run == -INFINITY) ? f32x2{-INFINITY, 0.0f} : f32x2{m_run * LN2, L};
+        if (w == 0 && g == 0) {
+            float lr = L;
+            if (m_run == -INFINITY && L != L && !any_live_key(a, t, k0, k1)) lr = 0.0f;
+            *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) = f32x2{(m_run == -INFINITY) ? -INFINITY : m_run * LN2, lr};
+        }
         if (m_run == -INFINITY) return;                      // no live key: the merge never reads this o
         d = reinterpret_cast<float *>(rec + part_o_off(a.n_split, sp, DV, 4)) + (size_t)hh * DV;
     }

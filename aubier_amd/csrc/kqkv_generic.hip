@@ -205,9 +205,11 @@ __global__ __launch_bounds__(256) void kqkv_generic_kernel(DecodeArgs a, int dk,
     char * rec = part_record(a.part, h / PART_HEADS, a.nt, t, a.n_split, dv, OB);
     const int hh = h % PART_HEADS;
     char * blk = rec + part_o_off(a.n_split, sp, dv, OB);
-    if (tid == 0)                    // l = 0 with no live key, also where masked keys left it NaN
-        *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) =
-            (m_run == -INFINITY) ? f32x2{-INFINITY, 0.0f} : f32x2{m_run * LN2, l_run};
+    if (tid == 0) {
+        float lr = l_run;
+        if (m_run == -INFINITY && l_run != l_run && !any_live_key(a, t, k0, k1)) lr = 0.0f;
+        *reinterpret_cast<f32x2 *>(rec + part_ml_off(a.n_split, hh, sp)) = f32x2{(m_run == -INFINITY) ? -INFINITY : m_run * LN2, lr};
+    }
     const float inv = l_run > 0.0f ? 1.0f / l_run : 0.0f;
     if (writer) {
         const f32x4 r = o * inv;
@@ -313,7 +315,7 @@ __global__ __launch_bounds__(256) void merge_rows_kernel(const char * __restrict
         f32x4 r = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 8; ++i) r += fold[i][tid >> 1][tid & 1];
-        const float inv = M == -INFINITY ? 0.0f : 1.0f / L;     // 0 only if every split is empty
+        const float inv = M == -INFINITY ? L : 1.0f / L;        // every split empty: 0 (NaN where a score was)
         *reinterpret_cast<f32x4 *>(dst + ((size_t)h * nt + t) * dv + blockIdx.x * MR_COLS + 4 * tid) = r * inv;
     }
 }
@@ -374,7 +376,7 @@ __global__ __launch_bounds__(256) void merge_few_kernel(const char * __restrict_
             for (int k = 0; k < 4; ++k) { O[k] += f * v0[k]; O[4 + k] += f * v1[k]; }
         }
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const float inv = L > 0.0f ? 1.0f / L : L;      // every split empty: 0 (NaN where a score was)
     float * d = dst + ((size_t)h * nt + t) * dv + 8 * c8;
     *reinterpret_cast<f32x4 *>(d) = f32x4{O[0] * inv, O[1] * inv, O[2] * inv, O[3] * inv};
     *reinterpret_cast<f32x4 *>(d + 4) = f32x4{O[4] * inv, O[5] * inv, O[6] * inv, O[7] * inv};

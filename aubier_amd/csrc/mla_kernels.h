@@ -16,7 +16,7 @@ namespace mla {
 //   m      a reference for the split's scores, natural-log units: the exact max (VALU kernel) or a
 //          running reference at most 15 ln 2 below it (MFMA kernels); -inf if the split is empty.
 //          The merge only uses m + ln l.
-//   l      sum_j exp(s_j - m)
+//   l      sum_j exp(s_j - m); NaN beside m = -inf where every live key's score is NaN
 //   o / l  the split's normalised softmax output.  T is the cache's element type: f16 for an f16
 //          cache (|o / l| <= max|V|, so it cannot overflow), f32 for f32.  A split with no live
 //          key (m = -inf) may leave its block unwritten; the merge never reads it.
@@ -53,6 +53,18 @@ struct DecodeArgs {
     char * part;            // partial blocks (when dst == null)
     float * dst;            // final output (single-split launches), contiguous [D_v, nt, H]
 };
+
+// Whether token t has a live key (mask > -inf) among keys [k0, k1).  For a record without a finite score
+// (m = -inf) whose l came out NaN: where live keys' scores were NaN l stays NaN, which the merge passes on;
+// where only masked cells were, which may hold anything, the split is empty and l is 0.
+__device__ __forceinline__ bool any_live_key(const DecodeArgs & a, int t, int k0, int k1) {
+    if (a.mask == nullptr) return k0 < k1;
+    const float * row = reinterpret_cast<const float *>(reinterpret_cast<const char *>(a.mask) + (size_t)t * a.mask_nb1);
+    bool live = false;
+#pragma unroll 8
+    for (int k = k0; k < k1; ++k) live |= row[k] != -INFINITY;
+    return live;
+}
 
 hipError_t launch_kqkv_decode_f16(int dk, int dv, const DecodeArgs & a, hipStream_t stream);
 // several query tokens (nt >= PREFILL_MIN_TOKENS, chunked prefill): 4 tokens per workgroup sharing

@@ -136,19 +136,17 @@ __device__ __forceinline__ void merge_unit(const char * __restrict__ part, int d
 #pragma unroll
         for (int i = 0; i < 4; ++i) M = fmaxf(M, sm[i][c8]);
         f32x4 r0 = {0.f, 0.f, 0.f, 0.f}, r1 = {0.f, 0.f, 0.f, 0.f};
-        if (M > -INFINITY) {
-            float LL = 0.0f;
+        float LL = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float f = exp2_unless(sm[i][c8] == -INFINITY, (sm[i][c8] - M) * LOG2E);
-                LL += sL[i][c8] * f;
-                r0 += sO[i][c8][0] * f;
-                r1 += sO[i][c8][1] * f;
-            }
-            const float inv = 1.0f / LL;
-            r0 *= inv;
-            r1 *= inv;
+        for (int i = 0; i < 4; ++i) {
+            const float f = exp2_unless(sm[i][c8] == -INFINITY, (sm[i][c8] - M) * LOG2E);
+            LL += sL[i][c8] * f;
+            r0 += sO[i][c8][0] * f;
+            r1 += sO[i][c8][1] * f;
         }
+        const float inv = M == -INFINITY ? LL : 1.0f / LL;      // every split empty: 0 (NaN where a score was)
+        r0 *= inv;
+        r1 *= inv;
         float * d = dst + ((size_t)h * nt + t) * dv + c;
         *reinterpret_cast<f32x4 *>(d) = r0;
         *reinterpret_cast<f32x4 *>(d + 4) = r1;

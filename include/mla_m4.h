@@ -207,7 +207,7 @@ int mla_m4_kqkv_partial(const mla_m4_tensor * kcache, const mla_m4_tensor * q,
  * GGML_OP_M4_PHASE, phase MLA_M4_PHASE_MERGE -- the split-K merge (the combine kernel of
  * patches/ggml-m4/m4-kqkv.cu:314-338): m* = max m_s; l* = sum l_s e^(m_s - m*);
  * o* = sum o_s e^(m_s - m*) over splits with m_s > -inf; dst = o* / l*, or 0 if every split is
- * empty.
+ * empty.  (l_s = NaN beside m_s = -inf: every live key's score was NaN, and dst is NaN.)
  *   part F32 ne [MLA_M4_PART_FLOATS(D_v) or MLA_M4_PART_FLOATS_F32(D_v), n_split, nt, ceil(H / 32)]
  *   dst  F32 ne [D_v, nt, H] contiguous (H and D_v are taken from dst; the o type from ne[0])
  * ------------------------------------------------------------------------------------------- */
