@@ -1,7 +1,7 @@
 """Batch-of-N decode: N rows in one KQKV, each over its own region of one cache window (the
 engine's per-sequence regions: a row's mask is 0 on [base, base + len) and -inf elsewhere,
-engine/m1_layer.h:212-223, engine/m1_session.h:188-201).  N < 4 runs the decode kernels (one
-token per workgroup), N >= 4 the 4-token prefill kernel.
+engine/m1_layer.h:212-223, engine/m1_session.h:188-201).  Below 16 rows the
+decode kernels run (a split's rows share its workgroup), from 16 on the prefill kernel.
 
 CPU: the oracle's row s over the full masked window equals the oracle over the row's own cells
 with no mask (a size-independent restatement of what the mask means), and the f64 brute force.
